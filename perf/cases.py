@@ -86,10 +86,10 @@ def draw(rng):
         return dict(kind=kind, mx=_log_int(rng, 32, 160), my=_log_int(rng, 20, 128), mz=_log_int(rng, 16, 80),
                     blocks=rng.choice([2, 3, 4]), steps=rng.choice([2, 4]), precision=4)
     if kind == "gradients":
-        return dict(kind=kind, n=16 * _log_int(rng, 16, 512), weights=rng.choice(["gelu", "hswish"]))
+        return dict(kind=kind, n=16 * _log_int(rng, 16, 256), weights=rng.choice(["gelu", "hswish"]))
     if kind == "surrogate":
-        return dict(kind=kind, n=_log_int(rng, 2000, 2000000), weights=rng.choice(["gelu", "hswish"]))
-    return dict(kind=kind, n=_log_int(rng, 1000, 1500000))
+        return dict(kind=kind, n=_log_int(rng, 2000, 1500000), weights=rng.choice(["gelu", "hswish"]))
+    return dict(kind=kind, n=_log_int(rng, 1000, 1000000))
 
 
 def _flow_case(case, seed):
