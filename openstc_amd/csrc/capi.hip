@@ -369,6 +369,13 @@ void make_chem64(const ostc_param &p, ChemF64 &out) {
       out.act_mask |= 1u << l;
       out.rank[l] = out.n_act++;
     }
+  out.t_mid_min = 1e300;
+  out.t_mid_max = out.t_low_max = p.n_spec > 0 ? -1e300 : 1e300;
+  for (int i = 0; i < p.n_spec && i < kMaxSpec; ++i) {
+    out.t_mid_min = std::min(out.t_mid_min, p.t_mid[i]);
+    out.t_mid_max = std::max(out.t_mid_max, p.t_mid[i]);
+    out.t_low_max = std::max(out.t_low_max, p.t_low[i]);
+  }
   for (int i = 0; i < p.n_spec && i < kMaxSpec; ++i) {
     for (int r = 0; r < 2; ++r) {
       const double *c = r == 0 ? &p.low_temp_coeff[i * 7] : &p.high_temp_coeff[i * 7];
@@ -379,6 +386,115 @@ void make_chem64(const ostc_param &p, ChemF64 &out) {
     out.g_low[i] = c[0] * (1.0 - std::log(tt)) - 0.5 * c[1] * tt - c[2] * tt * tt / 6.0 -
                    c[3] * tt * tt * tt / 12.0 - c[4] * tt * tt * tt * tt * 0.05 + c[5] / tt - c[6];
   }
+}
+// The reduced tables (ChemRed): ok = 0 where the mechanism does not fit them.
+// Kept species: rows of the net stoichiometric matrix that are independent of
+// those already kept, taken from the end of the species list -- mechanisms
+// list their reactants first, so the dependent ones are the reactants, which
+// carry the largest rates (a trace species formed as a difference of large
+// ones would lose digits).
+void make_chem_red(const ostc_param &p, ChemRed &out) {
+  std::memset(&out, 0, sizeof(out));
+  if (p.n_spec != kRedSpec || p.n_reac < 1 || p.n_reac > kMaxReac) return;
+  const int ns = kRedSpec, nr = p.n_reac;
+  const auto nf = [&](int r, int l) { return p.stoi_f[r * kMaxSpec + l]; };
+  const auto nb = [&](int r, int l) { return p.stoi_b[r * kMaxSpec + l]; };
+  for (int r = 0; r < nr; ++r) {
+    int a = 0, b = 0;
+    for (int l = 0; l < ns; ++l) {
+      if (nf(r, l) < 0 || nb(r, l) < 0) return;
+      a += nf(r, l);
+      b += nb(r, l);
+    }
+    if (a > 3 || b > 3) return;
+  }
+  // row echelon form of the kept rows, each with its combination of kept
+  // rows, so that a dependent row's combination can be read off
+  std::vector<std::vector<double>> ech, comb;
+  std::vector<int> lead, kept, dep, rest;
+  std::vector<std::vector<double>> dep_comb;
+  for (int l = ns - 1; l >= 0; --l) {
+    bool reacts = false;
+    std::vector<double> row(nr), cmb(ns, 0.0);
+    for (int r = 0; r < nr; ++r) {
+      row[r] = nb(r, l) - nf(r, l);
+      reacts = reacts || nf(r, l) != 0 || nb(r, l) != 0;
+    }
+    if (!reacts) {
+      rest.push_back(l);
+      continue;
+    }
+    // row = sum of echelon rows * f + remainder
+    for (size_t e = 0; e < ech.size(); ++e) {
+      const double f = row[lead[e]];
+      if (f == 0) continue;
+      for (int r = 0; r < nr; ++r) row[r] -= f * ech[e][r];
+      for (int q = 0; q < ns; ++q) cmb[q] += f * comb[e][q];
+    }
+    int at = -1;
+    for (int r = 0; r < nr; ++r)
+      if (std::fabs(row[r]) > 1e-9 && (at < 0 || std::fabs(row[r]) > std::fabs(row[at]))) at = r;
+    if (at < 0) {
+      dep.push_back(l);
+      dep_comb.push_back(cmb);
+      continue;
+    }
+    // the new echelon row, scaled to a leading 1: (row l - combination) / row[at]
+    const double s = 1.0 / row[at];
+    std::vector<double> e(nr), c(ns);
+    for (int r = 0; r < nr; ++r) e[r] = std::fabs(row[r]) > 1e-9 ? row[r] * s : 0.0;
+    for (int q = 0; q < ns; ++q) c[q] = -cmb[q] * s;
+    c[l] += s;
+    ech.push_back(e);
+    comb.push_back(c);
+    lead.push_back(at);
+    kept.push_back(l);
+  }
+  if (kept.empty() || (int)kept.size() > kRedKept || (int)dep.size() > kRedDep) return;
+  const int nk = (int)kept.size(), nd = (int)dep.size();
+  size_t next = 0;
+  int slot_of[kRedSpec];
+  for (int s = 0; s < kRedKept; ++s) out.slot[s] = s < nk ? kept[s] : rest[next++];
+  for (int s = 0; s < kRedDep; ++s) out.slot[kRedKept + s] = s < nd ? dep[s] : rest[next++];
+  out.slot[kRedSlots] = rest[next];
+  for (int s = 0; s < ns; ++s) {
+    slot_of[out.slot[s]] = s;
+    out.mw[s] = p.mw[out.slot[s]];
+  }
+  // molar combination -> mass: omega_dep / mw_dep = sum c_q omega_q / mw_q
+  for (int d = 0; d < nd; ++d)
+    for (int k = 0; k < nk; ++k) out.lin[d][k] = dep_comb[d][kept[k]] * p.mw[dep[d]] / p.mw[kept[k]];
+  for (int r = 0; r < nr; ++r) {
+    ReacRed &q = out.reac[r];
+    q.A = p.A[r], q.b = p.b[r], q.Ea = p.Ea[r];
+    q.A2 = p.A2[r], q.b2 = p.b2[r], q.Ea2 = p.Ea2[r];
+    q.troe_alpha = p.troe_alpha[r];
+    q.troe_t1 = p.troe_t1[r], q.troe_t2 = p.troe_t2[r], q.troe_t3 = p.troe_t3[r];
+    q.type = p.reac_type[r];
+    q.order = p.reac_order[r];
+    unsigned side[2] = {0, 0};
+    int cnt[2] = {0, 0};
+    for (int l = 0; l < ns; ++l) {
+      q.eff[l] = p.third_body_coeff[r * kMaxSpec + l];
+      const int s = slot_of[l], n2[2] = {nf(r, l), nb(r, l)};
+      if (s < kRedSlots) {
+        q.nf[s] = n2[0];
+        q.nb[s] = n2[1];
+        if (s < kRedKept) {
+          q.dm[s] = n2[1] - n2[0];
+          if (n2[1] != n2[0]) q.net |= 1u << s;
+        }
+      }
+      for (int h = 0; h < 2; ++h)
+        for (int c = 0; c < n2[h]; ++c) side[h] |= (unsigned)l << (8 * cnt[h]++);
+    }
+    for (int h = 0; h < 2; ++h)
+      while (cnt[h] < 3) side[h] |= (unsigned)kRedOne << (8 * cnt[h]++);
+    q.left = side[0];
+    q.right = side[1];
+  }
+  out.n_reac = nr;
+  out.ok = 1;
 }
 }  // namespace ostc
 
@@ -429,6 +545,13 @@ int ostc_ctx_create(const ostc_param *param, ostc_ctx **out) {
     n_act = cf.n_act;
     e = hipMemcpy(reinterpret_cast<char *>(c->dev) + kChemF64Offset, &cf, sizeof(cf), hipMemcpyHostToDevice);
   }
+  bool red = false;
+  if (e == hipSuccess) {
+    ChemRed cr;
+    make_chem_red(*param, cr);
+    red = cr.ok != 0;
+    e = hipMemcpy(reinterpret_cast<char *>(c->dev) + kChemRedOffset, &cr, sizeof(cr), hipMemcpyHostToDevice);
+  }
   if (e == hipSuccess && n_act == 0 && param->mix_model == OSTC_FR && param->chem_src_method == 1) {
     ostc_ctx_destroy(c);
     return fail(OSTC_ERR_ARG, "finite-rate chemistry with EPI: no species takes part in a reaction");
@@ -454,6 +577,7 @@ int ostc_ctx_create(const ostc_param *param, ostc_ctx **out) {
   o.implicit_method = param->implicit_method;
   o.dplur_steps = param->dplur_inner_step;
   o.n_act = n_act;
+  o.red = red;
   // launch tuning of the DPLUR sweep: 0 sizes its k chunks from the device's
   // resident workgroup capacity; the environment can fix a workgroup target
   o.dplur_wg = 0;
@@ -1079,7 +1203,7 @@ int ostc_chem_plain_step(ostc_ctx *c, long n, const double *t, const double *p, 
                          double *dy, void *s) {
   if (!c || n < 0 || (n > 0 && (!t || !p || !y || !dt || !dy))) return fail(OSTC_ERR_ARG, "bad arguments");
   if (c->user_ns != 9 || c->host.n_reac <= 0) return fail(OSTC_ERR_ARG, "needs the 9-species mechanism");
-  return chem_plain_step(c->dev, c->host.n_spec, c->host.n_reac, n, t, p, y, dt, dy, S(s));
+  return chem_plain_step(c->dev, c->host.n_spec, c->host.n_reac, c->opts.red, n, t, p, y, dt, dy, S(s));
 }
 
 int ostc_chem_source_batch(ostc_ctx *c, long n, const double *rho, const double *t, const double *y, double *omega,
@@ -1198,6 +1322,7 @@ int ostc_surrogate_create(ostc_ctx *ctx, const ostc_surrogate_desc *desc, const 
   S.params = sur_params(*desc);
   S.n_params = ostc::sur_n_params(desc->n_out);
   S.max_batch = max_batch;
+  S.red = ctx->opts.red;
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&S.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || S.cus <= 0)
@@ -1330,7 +1455,8 @@ int ostc_chem_zone_step(ostc_ctx *c, ostc_zone *z, ostc_surrogate *s, int mode, 
   const long n = (long)z->desc.mx * z->desc.my * z->desc.mz;
   int st;
   if (mode == 0) {
-    st = fp64(z) ? ostc::zone_plain_chem(c->dev, z->vd, dy, S(strm)) : ostc::zone_plain_chem(c->dev, z->vf, dy, S(strm));
+    st = fp64(z) ? ostc::zone_plain_chem(c->dev, c->opts.red, z->vd, dy, S(strm))
+                 : ostc::zone_plain_chem(c->dev, c->opts.red, z->vf, dy, S(strm));
     return st ? fail(st, "plain chemistry launch failed") : OSTC_OK;
   }
   st = sur_ensure_fallback(s, n);

@@ -621,6 +621,77 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   });
 }
 
+// The same for mechanisms with reduced tables (ChemRed): one pass over the
+// reactions with the kept species' 48 sums in registers and concentrations and
+// Gibbs energies in LDS, a 6 x 6 factorisation, 48 numbers stored.  Bound by
+// FP64 issue and scalar-load waits at two waves per SIMD (199 VGPRs; three
+// waves spill 92 B a lane and measured the same): 4 740 vector and 1 080
+// scalar instructions a wave where the whole block takes 9 190 and 3 170.
+// 0.748 -> 0.489 ms on a laminar block of 1.77 M cells.
+template <typename R, int NT>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_chem_dq0_red(
+    ZoneView<R> z, const ostc_param *__restrict__ p) {
+  constexpr int NS = kRedSpec, K = kRedKept;
+  __shared__ ConcGibbs tab_mem[kRedEntries * 256];
+  const auto c = cell_index(z, 0);
+  if (!c.ok) return;
+  const int64_t id = z.idx(c.i, c.j, c.k), P = z.plane;
+  const ChemRed *ct = chem_red(p);
+  const R dt = z.dt[id];
+  const R sri = z.spectr[id] + z.spectr[P + id] + z.spectr[2 * P + id];
+  const R diag = (R)1 + dt * sri;
+  // flow and turbulence rows as k_dq0 forms them
+#pragma unroll
+  for (int l = 0; l < 5; ++l) z.dq0[l * P + id] = z.dq[l * P + id] / diag;
+  if constexpr (NT > 0) {
+    if (p->turb_implicit == 1) {
+      z.dq0[(NS + 5) * P + id] = z.dq[(NS + 5) * P + id] / (diag - dt * z.turb_jac[id]);
+      z.dq0[(NS + 6) * P + id] = z.dq[(NS + 6) * P + id] / (diag - dt * z.turb_jac[P + id]);
+    } else {
+      z.dq0[(NS + 5) * P + id] = z.dq[(NS + 5) * P + id] / diag;
+      z.dq0[(NS + 6) * P + id] = z.dq[(NS + 6) * P + id] / diag;
+    }
+  }
+  double a[K * K], cc[K * kRedDep], om[K];
+  int piv[K];
+  {
+    R y[NS];
+#pragma unroll
+    for (int l = 0; l < NS; ++l) y[l] = z.sv[l * P + id];
+    double zz[kRedFactors];
+    chem_red_source(p, (double)z.bv[id], (double)z.bv[5 * P + id], [&](int l) { return (double)y[l]; },
+                    tab_mem + threadIdx.x + 64 * threadIdx.y, 256, zz, om);
+    chem_red_factor(ct, zz, (double)dt, (double)diag, a, cc, piv);
+  }
+  unsigned w = 0;
+#pragma unroll
+  for (int q = 0; q < K * K; ++q) z.chem_lu[lu_tiled(id, q, kRedFactors)] = a[q];
+#pragma unroll
+  for (int q = 0; q < K * kRedDep; ++q) z.chem_lu[lu_tiled(id, K * K + q, kRedFactors)] = cc[q];
+#pragma unroll
+  for (int q = 0; q < K; ++q) w |= (unsigned)piv[q] << (4 * q);
+  z.chem_piv[id] = (int)w;
+  // the species rows of dq with the source added, at the bulk precision
+  const R J = z.jac[id];
+  double b[kRedSlots];
+#pragma unroll
+  for (int m = 0; m < kRedSlots; ++m) {
+    double o = 0;
+    if (m < K)
+      o = om[m < K ? m : 0];
+    else
+#pragma unroll
+      for (int n = 0; n < K; ++n) o += ct->lin[m - K][n] * om[n];
+    b[m] = (double)(z.dq[(5 + ct->slot[m]) * P + id] + (R)((double)J * o));
+  }
+  const double inv_diag = 1.0 / (double)diag;
+  chem_red_solve(ct, a, cc, piv, inv_diag, b);
+#pragma unroll
+  for (int m = 0; m < kRedSlots; ++m) z.dq0[(5 + ct->slot[m]) * P + id] = (R)b[m];
+  const int64_t q = (5 + ct->slot[kRedSlots]) * P + id;
+  z.dq0[q] = (R)((double)z.dq[q] * inv_diag);
+}
+
 // Diagonal solve and write of one cell after a DPLUR sweep has gathered its
 // off-diagonal sum acc (src/DPLURHPP.cuh:193-249); EPI_for_dqk
 // (src/FiniteRateChem.cu:255-284) with the LU factors from k_dq0.  FIRST
@@ -711,6 +782,41 @@ __global__ __launch_bounds__(256) void k_dplur_chem(ZoneView<R> z, const ostc_pa
       if (ct->rank[m] < 0)
         dout[(5 + m) * P + id] = (R)((double)z.dq0[(5 + m) * P + id] + (double)dout[(5 + m) * P + id] * dtd / dg);
   }
+}
+
+// The same with the reduced factors of k_chem_dq0_red: 48 numbers a cell
+// instead of 64.  HBM-bound: 512 B a cell instead of 640, 0.222 -> 0.185 ms on
+// a block of 1.77 M cells (4.9 TB/s).
+template <typename R>
+__global__ __launch_bounds__(256) void k_dplur_chem_red(ZoneView<R> z, const ostc_param *__restrict__ p,
+                                                        R *__restrict__ dout) {
+  constexpr int K = kRedKept;
+  const auto c = cell_index(z, 0);
+  if (!c.ok) return;
+  const int64_t id = z.idx(c.i, c.j, c.k), P = z.plane;
+  const ChemRed *ct = chem_red(p);
+  double a[K * K], cc[K * kRedDep], b[kRedSlots];
+  int piv[K];
+#pragma unroll
+  for (int q = 0; q < K * K; ++q) a[q] = z.chem_lu[lu_tiled(id, q, kRedFactors)];
+#pragma unroll
+  for (int q = 0; q < K * kRedDep; ++q) cc[q] = z.chem_lu[lu_tiled(id, K * K + q, kRedFactors)];
+  const unsigned w = (unsigned)z.chem_piv[id];
+#pragma unroll
+  for (int q = 0; q < K; ++q) piv[q] = (int)(w >> (4 * q) & 15u);
+  const R dt = z.dt[id];
+  const double dtd = (double)dt;
+  const double inv_diag = 1.0 / (double)((R)1 + dt * (z.spectr[id] + z.spectr[P + id] + z.spectr[2 * P + id]));
+#pragma unroll
+  for (int m = 0; m < kRedSlots; ++m) b[m] = (double)dout[(5 + ct->slot[m]) * P + id] * dtd;
+  chem_red_solve(ct, a, cc, piv, inv_diag, b);
+#pragma unroll
+  for (int m = 0; m < kRedSlots; ++m) {
+    const int64_t q = (5 + ct->slot[m]) * P + id;
+    dout[q] = (R)((double)z.dq0[q] + b[m]);
+  }
+  const int64_t q = (5 + ct->slot[kRedSlots]) * P + id;
+  dout[q] = (R)((double)z.dq0[q] + (double)dout[q] * dtd * inv_diag);
 }
 
 // Per-cell inputs of the convective-Jacobian products of one DPLUR sweep
@@ -1636,7 +1742,11 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
     if (chem) {
       if (o.ns == 9 && o.chem == 1 && chem_late) {
         // the chemistry after the fluxes, with dq0 (chem_after_fluxes)
-        if (o.nt == 2)
+        if (o.red && o.nt == 2)
+          hipLaunchKernelGGL((k_chem_dq0_red<R, 2>), g.grid, g.block, 0, st, z, dp);
+        else if (o.red)
+          hipLaunchKernelGGL((k_chem_dq0_red<R, 0>), g.grid, g.block, 0, st, z, dp);
+        else if (o.nt == 2)
           hipLaunchKernelGGL((k_chem_dq0<R, 2>), g.grid, g.block, 0, st, z, dp);
         else
           hipLaunchKernelGGL((k_chem_dq0<R, 0>), g.grid, g.block, 0, st, z, dp);
@@ -1701,7 +1811,9 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
       prof_mark(P_DPLUR_CHEM, st, true);
       if (o.ns == 9) {
         // factors stored by the source kernel are tiled (lu_tiled)
-        if (chem_late)
+        if (chem_late && o.red)
+          hipLaunchKernelGGL((k_dplur_chem_red<R>), g.grid, g.block, 0, st, z, dp, out);
+        else if (chem_late)
           OSTC_DISPATCH_NA(o, hipLaunchKernelGGL((k_dplur_chem<R, 9, NA_, true>), g.grid, g.block, 0, st, z, dp, out));
         else
           OSTC_DISPATCH_NA(o, hipLaunchKernelGGL((k_dplur_chem<R, 9, NA_>), g.grid, g.block, 0, st, z, dp, out));

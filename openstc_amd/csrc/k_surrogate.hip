@@ -485,12 +485,13 @@ __global__ __launch_bounds__(256) void k_sur_decode(SurParams s, Src src, InferO
 // Plain point-implicit step on the fallback sub-lists (grid-stride over their
 // total, which lives on the device; entry q is found by a binary search over
 // the sub-list offsets).
-template <typename Src>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_sur_fallback(
+template <typename Src, bool RED>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_sur_fallback(
     const ostc_param *__restrict__ p, Src src,
                                                       const int *__restrict__ count, const long *__restrict__ list,
                                                       long cap, double *__restrict__ dyo) {
   __shared__ int pre[kFbLists + 1];
+  __shared__ ConcGibbs tab_mem[RED ? kRedEntries * 64 : 1];
   for (int l = threadIdx.x; l < kFbLists; l += blockDim.x) pre[l + 1] = count[l * kFbStride];
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -509,21 +510,34 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void
         hi = mid;
     }
     const long c = list[lo * cap + (q - pre[lo])];
-    double T, P, DT, Y[kNs], dy[kNs];
+    double T, P, DT, Y[kNs];
     src.load(c, T, P, Y, DT);
-    plain_chem_step<kNs>(p, T, P, Y, DT, dy);
+    if constexpr (RED) {
+      plain_chem_step_red(p, T, P, Y, DT, tab_mem + threadIdx.x, 64,
+                          [&](int k, double v) { dyo[c * kNs + k] = v; });
+    } else {
+      double dy[kNs];
+      plain_chem_step<kNs>(p, T, P, Y, DT, dy);
 #pragma unroll
-    for (int k = 0; k < kNs; ++k) dyo[c * kNs + k] = dy[k];
+      for (int k = 0; k < kNs; ++k) dyo[c * kNs + k] = dy[k];
+    }
   }
 }
 
-template <typename Src>
-__global__ __launch_bounds__(256) void k_zone_plain(const ostc_param *__restrict__ p, Src src,
-                                                    double *__restrict__ dyo) {
+template <typename Src, bool RED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_zone_plain(
+    const ostc_param *__restrict__ p, Src src, double *__restrict__ dyo) {
+  __shared__ ConcGibbs tab_mem[RED ? kRedEntries * 256 : 1];
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= src.n) return;
-  double T, P, DT, Y[kNs], dy[kNs];
+  double T, P, DT, Y[kNs];
   src.load(c, T, P, Y, DT);
+  if constexpr (RED) {
+    plain_chem_step_red(p, T, P, Y, DT, tab_mem + threadIdx.x, 256,
+                        [&](int k, double v) { dyo[c * kNs + k] = v; });
+    return;
+  }
+  double dy[kNs];
   plain_chem_step<kNs>(p, T, P, Y, DT, dy);
 #pragma unroll
   for (int k = 0; k < kNs; ++k) dyo[c * kNs + k] = dy[k];
@@ -740,8 +754,13 @@ static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, 
   // spread a typical fallback list over every CU; the kernel strides over
   // the device-side count
   const long fb_blocks = std::min<long>((src.n + 63) / 64, 16L * st.cus);
-  hipLaunchKernelGGL(k_sur_fallback<Src>, dim3((unsigned)std::max<long>(1, fb_blocks)), dim3(64), 0, s, dp, src,
-                     st.fb_count, st.fb_list, fb_list_cap(st.fb_cap), dy);
+  const dim3 fb_grid((unsigned)std::max<long>(1, fb_blocks));
+  if (st.red)
+    hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.fb_count, st.fb_list,
+                       fb_list_cap(st.fb_cap), dy);
+  else
+    hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.fb_count, st.fb_list,
+                       fb_list_cap(st.fb_cap), dy);
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
@@ -759,9 +778,13 @@ int sur_infer_zone(const SurState &st, const ostc_param *dp, const ZoneView<R> &
 }
 
 template <typename R>
-int zone_plain_chem(const ostc_param *dp, const ZoneView<R> &z, double *dy, hipStream_t s) {
+int zone_plain_chem(const ostc_param *dp, bool red, const ZoneView<R> &z, double *dy, hipStream_t s) {
   ZoneSrc<R> src{z.bv, z.sv, z.dt, z.mx, z.my, z.g, z.nx, z.ny, z.plane, (long)z.mx * z.my * z.mz};
-  hipLaunchKernelGGL(k_zone_plain<ZoneSrc<R>>, dim3((unsigned)((src.n + 255) / 256)), dim3(256), 0, s, dp, src, dy);
+  const dim3 grid((unsigned)((src.n + 255) / 256)), block(256);
+  if (red)
+    hipLaunchKernelGGL((k_zone_plain<ZoneSrc<R>, true>), grid, block, 0, s, dp, src, dy);
+  else
+    hipLaunchKernelGGL((k_zone_plain<ZoneSrc<R>, false>), grid, block, 0, s, dp, src, dy);
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
@@ -769,8 +792,8 @@ template int sur_infer_zone<float>(const SurState &, const ostc_param *, const Z
                                    hipStream_t);
 template int sur_infer_zone<double>(const SurState &, const ostc_param *, const ZoneView<double> &, double *,
                                     hipStream_t);
-template int zone_plain_chem<float>(const ostc_param *, const ZoneView<float> &, double *, hipStream_t);
-template int zone_plain_chem<double>(const ostc_param *, const ZoneView<double> &, double *, hipStream_t);
+template int zone_plain_chem<float>(const ostc_param *, bool, const ZoneView<float> &, double *, hipStream_t);
+template int zone_plain_chem<double>(const ostc_param *, bool, const ZoneView<double> &, double *, hipStream_t);
 
 int sur_gradients(const SurState &st, long nb, const double *t, const double *p, const double *y, const double *dt,
                   const int *idx, const float *target, float *grad, double *loss_dev, hipStream_t s) {

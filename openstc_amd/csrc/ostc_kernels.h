@@ -41,6 +41,7 @@ struct CellOpts {
   int rans_model, turb_implicit, implicit_method, dplur_steps;
   int dplur_wg;            // DPLUR sweep workgroup target (launch tuning; 0 = from the resident capacity)
   int n_act;               // species that take part in a reaction (the EPI block's size)
+  bool red;                // the mechanism has reduced chemistry tables (ChemRed)
 };
 template <typename R>
 int cv_from_bv(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st);
@@ -62,11 +63,12 @@ template <typename R>
 int source_terms(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool force,
                  bool *wrote, bool with_dt = false);
 inline bool source_has_dt(const CellOpts &o) { return o.nt > 0 && o.mix_model != OSTC_FR; }
-// EPI chemistry under DPLUR on the 9-species kernels with the two-pass
-// chemistry (at most 20 reactions)
+// EPI chemistry under DPLUR on the 9-species kernels: mechanisms with reduced
+// chemistry tables, and of the others those the two-pass chemistry takes (at
+// most 20 reactions)
 inline bool chem_after_fluxes(const CellOpts &o) {
-  return o.mix_model == OSTC_FR && o.chem == 1 && o.implicit_method == 1 && o.ns == 9 && o.n_reac <= 20 &&
-         o.n_act > 0;
+  return o.mix_model == OSTC_FR && o.chem == 1 && o.implicit_method == 1 && o.ns == 9 &&
+         (o.red || (o.n_reac <= 20 && o.n_act > 0));
 }
 template <typename R>
 int local_time_step(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st);
@@ -108,7 +110,8 @@ template <typename R>
 int wall_friction_heatflux(const ZoneView<R> &z, double dyn_pressure, double *cf, double *qw, hipStream_t st);
 
 // k_chem.hip
-int chem_plain_step(const ostc_param *dp, int ns, int nr, long n, const double *t, const double *p, const double *y,
+// red: the mechanism has reduced tables (ChemRed)
+int chem_plain_step(const ostc_param *dp, int ns, int nr, bool red, long n, const double *t, const double *p, const double *y,
                     const double *dt, double *dy, hipStream_t st);
 int chem_source_batch(const ostc_param *dp, int ns, int nr, long n, const double *rho, const double *t,
                       const double *y, double *omega, double *jac, hipStream_t st);

@@ -60,6 +60,7 @@ struct SurParams {
 struct SurState {
   SurParams params{};
   int n_params = 0;
+  bool red = false;  // the mechanism has reduced chemistry tables (fallback step)
   int cus = 256;
   long max_batch = 0;
   long adam_step = 0;
@@ -128,7 +129,7 @@ int sur_infer_batch(const SurState &st, const ostc_param *dp, long n, const doub
 template <typename R>
 int sur_infer_zone(const SurState &st, const ostc_param *dp, const ZoneView<R> &z, double *dy, hipStream_t s);
 template <typename R>
-int zone_plain_chem(const ostc_param *dp, const ZoneView<R> &z, double *dy, hipStream_t s);
+int zone_plain_chem(const ostc_param *dp, bool red, const ZoneView<R> &z, double *dy, hipStream_t s);
 int sur_gradients(const SurState &st, long nb, const double *t, const double *p, const double *y, const double *dt,
                   const int *idx, const float *target, float *grad, double *loss_dev, hipStream_t s);
 int sur_adam(SurState &st, float lr, hipStream_t s);

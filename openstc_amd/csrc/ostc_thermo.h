@@ -55,6 +55,7 @@ struct ChemF64 {
   // + c6 / T; below T_low the value at T_low
   double g[2][kMaxSpec][7];
   double g_low[kMaxSpec];
+  double t_mid_min, t_mid_max, t_low_max;  // over the species: the wave-uniform range test
   // species that take part in at least one reaction, in order: act[r] is the
   // r-th of them, rank[k] species k's position among them (-1: none -- its
   // row and column of the EPI Jacobian are zero), n_act their count
@@ -68,7 +69,52 @@ struct ChemF64 {
   int jr[kMaxSpec][kMaxReac];
 };
 constexpr size_t kChemF64Offset = (kThermoF32Offset + sizeof(ThermoF32) + 255) / 256 * 256;
-constexpr size_t kParamBlockBytes = kChemF64Offset + sizeof(ChemF64);
+// The chemistry of a mechanism reduced by its conserved elements.  A reaction
+// moves atoms between species, so the production rates (and every column of
+// the EPI Jacobian J) of the species that react lie in the space the net
+// stoichiometric vectors span: of n_act rows only rank(net) are independent,
+// the others are fixed combinations of them, J_dep = L J_kept (L constant).
+// With the conserved elements taken out, the block (diag I - dt J) x = b is
+//   A x_kept = b_kept + C u,  u = (b_dep - L b_kept) / diag,
+//   x_dep = L x_kept + u,     A = diag I - dt (J_kk + J_kd L),  C = dt J_kd:
+// H2-air (9 species, 8 of them reacting, elements H and O) leaves a 6 x 6
+// matrix and a 6 x 2 one, 48 numbers a cell, where the whole block has 64, and
+// 6 of the 9 rows of sums.  The tables below are in slot order: slots 0..5 the
+// kept species, 6..7 the dependent ones, 8 a species that does not react.  A
+// mechanism with fewer of either fills the remaining slots with species that
+// do not react (zero rows and columns of J, a zero row of L); it has enough of
+// those, since 9 - n_act >= (6 - kept) + (2 - dependent) + 1 for n_act <= 8.
+constexpr int kRedKept = 6, kRedDep = 2, kRedSlots = kRedKept + kRedDep, kRedSpec = 9;
+constexpr int kRedFactors = kRedKept * kRedSlots;  // stored per cell: A's factors, then C
+constexpr int kRedOne = kRedSpec;                  // table entry with c = 1, g = 0
+struct ReacRed {
+  double A, b, Ea, A2, b2, Ea2;
+  double troe_alpha, troe_t1, troe_t2, troe_t3;
+  double nf[kRedSlots], nb[kRedSlots];  // stoichiometric coefficients by slot
+  double dm[kRedKept];                  // nb - nf of the kept slots
+  double eff[kRedSpec];                 // third-body efficiencies by species
+  int type, order;
+  // up to three reactants and three products (a coefficient of 2 twice) as
+  // species numbers in bytes, filled up with kRedOne
+  unsigned left, right;
+  unsigned net;  // bit m: dm[m] != 0
+  int pad[3];
+};
+struct ChemRed {
+  int ok;               // the mechanism fits these tables
+  int n_reac;
+  int slot[kRedSpec];   // species number of each slot
+  int pad;
+  double lin[kRedDep][kRedKept];  // L
+  double mw[kRedSpec];            // by slot
+  ReacRed reac[kMaxReac];
+};
+constexpr size_t kChemRedOffset = (kChemF64Offset + sizeof(ChemF64) + 255) / 256 * 256;
+constexpr size_t kParamBlockBytes = kChemRedOffset + sizeof(ChemRed);
+__host__ __device__ __forceinline__ const ChemRed *chem_red(const ostc_param *p) {
+  return reinterpret_cast<const ChemRed *>(reinterpret_cast<const char *>(p) + kChemRedOffset);
+}
+void make_chem_red(const ostc_param &p, ChemRed &out);
 __host__ __device__ __forceinline__ const ChemF64 *chem64(const ostc_param *p) {
   return reinterpret_cast<const ChemF64 *>(reinterpret_cast<const char *>(p) + kChemF64Offset);
 }
@@ -383,6 +429,18 @@ template <int NS>
 __device__ __forceinline__ void gibbs_div_rt(double t, double log_t, double t_inv, const ostc_param *__restrict__ p,
                                              double *g) {
   const ChemF64 *ct = chem64(p);
+  // one range for the whole wave: the coefficients are scalar operands (the
+  // same expression on the same numbers, without the per-lane choice)
+  const bool above = t >= ct->t_low_max;
+  const int row = __all(above && t >= ct->t_mid_max) ? 1 : (__all(above && t < ct->t_mid_min) ? 0 : -1);
+  if (row >= 0) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const double *c = ct->g[row][i];
+      g[i] = c[0] + c[1] * log_t + t * (c[2] + t * (c[3] + t * (c[4] + t * c[5]))) + c[6] * t_inv;
+    }
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < NS; ++i) {
     const bool hi = t >= p->t_mid[i];
@@ -903,6 +961,234 @@ __device__ __forceinline__ void lu_solve_any(const double *a, const int *piv, do
     lu_solve<NS>(a, piv, b, NS);
 }
 
+// ------------------------------------------------- reduced chemistry (ChemRed)
+// Concentrations c [mol/cm3] and g/RT of the 9 species and the filler entry
+// (1, 0) of each thread, in LDS: entry e at tab[e * stride], so that a
+// reaction reads its reactants and products by number, one 16-byte read each,
+// without a branch per species.
+struct ConcGibbs {
+  double c, g;
+};
+constexpr int kRedEntries = kRedSpec + 1;
+
+// J (kept rows, unscaled sums of dm * (nf q1 - nb q2)) and production sums of
+// the kept species, one pass over the reactions (sums in reaction order, as
+// the other forms): src/FiniteRateChem.cu:7-209.  The rate law is
+// reaction_rates', on the table.
+__device__ __forceinline__ void chem_red_sums(const ChemRed *__restrict__ ct, const ConcGibbs *tab, int stride,
+                                              double t, double t_inv, double log_t, double *zz, double *om) {
+  const double temp_t = kPatm / kRu * 1e-3 * t_inv, temp_t_inv = 1.0 / temp_t;
+#pragma unroll
+  for (int q = 0; q < kRedFactors; ++q) zz[q] = 0;
+#pragma unroll
+  for (int m = 0; m < kRedKept; ++m) om[m] = 0;
+  const int nr = ct->n_reac;
+#pragma unroll 1
+  for (int r = 0; r < nr; ++r) {
+    const ReacRed &rc = ct->reac[r];
+    const int type = rc.type;
+    const unsigned left = rc.left, right = rc.right;
+    const ConcGibbs *l0 = tab + (left & 255) * stride, *l1 = tab + (left >> 8 & 255) * stride,
+                    *l2 = tab + (left >> 16) * stride;
+    const ConcGibbs *r0 = tab + (right & 255) * stride, *r1 = tab + (right >> 8 & 255) * stride,
+                    *r2 = tab + (right >> 16) * stride;
+    double kf = rc.A * exp(rc.b * log_t - rc.Ea * t_inv);
+    double kb;
+    if (type == 2) {
+      kb = rc.A2 * exp(rc.b2 * log_t - rc.Ea2 * t_inv);
+    } else {
+      // kf / Kc over kf, Kc = temp_t^order * exp(-d_gibbs)
+      const double d_gibbs = r0->g + r1->g + r2->g - (l0->g + l1->g + l2->g);
+      kb = exp(d_gibbs);
+      const int order = rc.order;
+      const double base = order >= 0 ? temp_t_inv : temp_t;
+      for (int q = 0; q < (order >= 0 ? order : -order); ++q) kb *= base;
+      if (type == 3) {
+        kf += rc.A2 * exp(rc.b2 * log_t - rc.Ea2 * t_inv);
+      } else if (type > 3) {
+        double cc = 0;
+#pragma unroll
+        for (int l = 0; l < kRedSpec; ++l) cc += tab[l * stride].c * rc.eff[l];
+        if (type == 4) {
+          kf *= cc;
+        } else {
+          const double kf_low = rc.A2 * exp(rc.b2 * log_t - rc.Ea2 * t_inv);
+          const double pr = kf_low * cc / kf;
+          double fv = 1.0;
+          if (type > 5) {
+            double f_cent = (1 - rc.troe_alpha) * exp(-t / rc.troe_t3) + rc.troe_alpha * exp(-t / rc.troe_t1);
+            if (type == 7) f_cent += exp(-rc.troe_t2 * t_inv);
+            const double logFc = log10(f_cent);
+            const double cc1 = -0.4 - 0.67 * logFc;
+            const double n = 0.75 - 1.27 * logFc;
+            const double logPr = log10(pr);
+            const double tempo = (logPr + cc1) / (n - 0.14 * (logPr + cc1));
+            fv = exp10(logFc / (1.0 + tempo * tempo));
+          }
+          kf = kf * pr / (1.0 + pr) * fv;
+        }
+      }
+      kb *= kf;
+    }
+    // the concentrations are read only now: held through the rate law they
+    // would cost 24 registers
+    __builtin_amdgcn_sched_barrier(0);
+    const double q1 = kf * l0->c * l1->c * l2->c, q2 = kb * r0->c * r1->c * r2->c;
+    const double dq = q1 - q2;
+    double v[kRedSlots];
+#pragma unroll
+    for (int n = 0; n < kRedSlots; ++n) v[n] = rc.nf[n] * q1 - rc.nb[n] * q2;
+    const unsigned net = rc.net;
+#pragma unroll
+    for (int m = 0; m < kRedKept; ++m) {
+      if (net & (1u << m)) {
+        const double dm = rc.dm[m];
+        om[m] += dm * dq;
+#pragma unroll
+        for (int n = 0; n < kRedSlots; ++n) zz[m * kRedSlots + n] += dm * v[n];
+      }
+    }
+  }
+}
+
+// The table of one thread and the sums above from (rho, T, Y); y(l) returns
+// the mass fraction of species l.  On return zz holds J's kept rows (1/s) and
+// om the production rates [kg/m3/s] of the kept species.
+template <class YOf>
+__device__ __forceinline__ void chem_red_source(const ostc_param *__restrict__ p, double rho, double t, YOf y,
+                                                ConcGibbs *tab, int stride, double *zz, double *om) {
+  const ChemRed *ct = chem_red(p);
+  const ChemF64 *cf = chem64(p);
+  const double log_t = log(t), t_inv = 1.0 / t;
+  {
+    double g[kRedSpec];
+    gibbs_div_rt<kRedSpec>(t, log_t, t_inv, p, g);
+#pragma unroll
+    for (int l = 0; l < kRedSpec; ++l) tab[l * stride] = {rho * y(l) * cf->inv_mw[l] * 1e-3, g[l]};
+    tab[kRedOne * stride] = {1.0, 0.0};
+  }
+  chem_red_sums(ct, tab, stride, t, t_inv, log_t, zz, om);
+  // J_mn = mw_m sum_mn / (rho Y_n) * 1e3 with rho Y_n = c_n mw_n 1e3, zero
+  // where Y_n <= 1e-25
+  const double tiny = 1e-25 * rho;
+#pragma unroll
+  for (int n = 0; n < kRedSlots; ++n) {
+    const double ry = tab[ct->slot[n] * stride].c * (ct->mw[n] * 1e+3);
+    const bool on = ry > tiny;
+    const double f = on ? 1e+3 / ry : 0.0;
+#pragma unroll
+    for (int m = 0; m < kRedKept; ++m) zz[m * kRedSlots + n] = on ? ct->mw[m] * (zz[m * kRedSlots + n] * f) : 0.0;
+  }
+#pragma unroll
+  for (int m = 0; m < kRedKept; ++m) om[m] *= ct->mw[m] * 1e+3;
+}
+
+// zz (J's kept rows) -> A's factors in a (36, diagonal of U inverted), C in
+// c (12) and the pivots
+__device__ __forceinline__ void chem_red_factor(const ChemRed *__restrict__ ct, const double *zz, double dt,
+                                                double diag, double *a, double *c, int *piv) {
+  constexpr int K = kRedKept;
+#pragma unroll
+  for (int m = 0; m < K; ++m) {
+#pragma unroll
+    for (int d = 0; d < kRedDep; ++d) c[m * kRedDep + d] = dt * zz[m * kRedSlots + K + d];
+#pragma unroll
+    for (int n = 0; n < K; ++n) {
+      double v = zz[m * kRedSlots + n];
+#pragma unroll
+      for (int d = 0; d < kRedDep; ++d) v += zz[m * kRedSlots + K + d] * ct->lin[d][n];
+      a[m * K + n] = (m == n ? diag : 0.0) - dt * v;
+    }
+  }
+#pragma unroll
+  for (int n = 0; n < K; ++n) {
+    int ik = n;
+    double best = 0;
+#pragma unroll
+    for (int m = n; m < K; ++m) {
+      double v = a[m * K + n];
+#pragma unroll
+      for (int q = 0; q < n; ++q) v -= a[m * K + q] * a[q * K + n];
+      a[m * K + n] = v;
+      if (m == n) {
+        best = fabs(v);
+      } else if (fabs(v) > best) {
+        best = fabs(v);
+        ik = m;
+      }
+    }
+    piv[n] = ik;
+#pragma unroll
+    for (int m = n + 1; m < K; ++m) {
+      const bool sw = ik == m;
+#pragma unroll
+      for (int q = 0; q < K; ++q) {
+        const double x = a[m * K + q], y = a[n * K + q];
+        a[m * K + q] = sw ? y : x;
+        a[n * K + q] = sw ? x : y;
+      }
+    }
+#pragma unroll
+    for (int q = n + 1; q < K; ++q) {
+      double v = a[n * K + q];
+#pragma unroll
+      for (int s = 0; s < n; ++s) v -= a[n * K + s] * a[s * K + q];
+      a[n * K + q] = v;
+    }
+    const double inv = 1.0 / a[n * K + n];
+    a[n * K + n] = inv;
+#pragma unroll
+    for (int m = n + 1; m < K; ++m) a[m * K + n] *= inv;
+  }
+}
+
+// x = (diag I - dt J)^-1 b of the 8 slots in place (b[0..5] kept, b[6..7]
+// dependent)
+__device__ __forceinline__ void chem_red_solve(const ChemRed *__restrict__ ct, const double *a, const double *c,
+                                               const int *piv, double inv_diag, double *b) {
+  constexpr int K = kRedKept;
+  double u[kRedDep];
+#pragma unroll
+  for (int d = 0; d < kRedDep; ++d) {
+    double v = b[K + d];
+#pragma unroll
+    for (int n = 0; n < K; ++n) v -= ct->lin[d][n] * b[n];
+    u[d] = v * inv_diag;
+  }
+#pragma unroll
+  for (int m = 0; m < K; ++m)
+#pragma unroll
+    for (int d = 0; d < kRedDep; ++d) b[m] += c[m * kRedDep + d] * u[d];
+#pragma unroll
+  for (int m = 0; m < K - 1; ++m) {
+    const int s = piv[m];
+#pragma unroll
+    for (int r = m + 1; r < K; ++r) {
+      const bool sw = s == r;
+      const double x = b[r], y = b[m];
+      b[r] = sw ? y : x;
+      b[m] = sw ? x : y;
+    }
+  }
+#pragma unroll
+  for (int m = 1; m < K; ++m)
+#pragma unroll
+    for (int q = 0; q < m; ++q) b[m] -= a[m * K + q] * b[q];
+#pragma unroll
+  for (int m = K - 1; m >= 0; --m) {
+#pragma unroll
+    for (int q = m + 1; q < K; ++q) b[m] -= a[m * K + q] * b[q];
+    b[m] *= a[m * K + m];
+  }
+#pragma unroll
+  for (int d = 0; d < kRedDep; ++d) {
+    double v = u[d];
+#pragma unroll
+    for (int n = 0; n < K; ++n) v += ct->lin[d][n] * b[n];
+    b[K + d] = v;
+  }
+}
+
 // The plain point-implicit chemistry step at fixed (T, p):
 // (I - dt*J) d(rhoY) = dt*omega, dY = d(rhoY)/rho -- the reference's explicit
 // EPI (src/FiniteRateChem.cu:211-234) applied to the chemical source alone.
@@ -931,6 +1217,37 @@ __device__ __forceinline__ void plain_chem_step(const ostc_param *__restrict__ p
   lu_solve<NS>(a, piv, om, NS);
 #pragma unroll
   for (int l = 0; l < NS; ++l) dy[l] = om[l] / rho;
+}
+
+// The same step on the reduced tables: out(k, dY_k) receives the changes.
+template <class Out>
+__device__ __forceinline__ void plain_chem_step_red(const ostc_param *__restrict__ p, double tc, double pc,
+                                                    const double *yy, double dtc, ConcGibbs *tab, int stride,
+                                                    Out out) {
+  const ChemRed *ct = chem_red(p);
+  double mw = 0;
+#pragma unroll
+  for (int l = 0; l < kRedSpec; ++l) mw += yy[l] / p->mw[l];
+  mw = 1 / mw;
+  const double rho = pc * mw / (kRu * tc);
+  double zz[kRedFactors], a[kRedKept * kRedKept], c[kRedKept * kRedDep], b[kRedSlots];
+  int piv[kRedKept];
+  chem_red_source(p, rho, tc, [&](int l) { return yy[l]; }, tab, stride, zz, b);
+  chem_red_factor(ct, zz, dtc, 1.0, a, c, piv);
+#pragma unroll
+  for (int m = 0; m < kRedKept; ++m) b[m] *= dtc;
+  // the dependent rows of dt * omega: L times the kept ones
+#pragma unroll
+  for (int d = 0; d < kRedDep; ++d) {
+    b[kRedKept + d] = 0;
+#pragma unroll
+    for (int n = 0; n < kRedKept; ++n) b[kRedKept + d] += ct->lin[d][n] * b[n];
+  }
+  chem_red_solve(ct, a, c, piv, 1.0, b);
+  const double rinv = 1.0 / rho;
+#pragma unroll
+  for (int m = 0; m < kRedSlots; ++m) out(ct->slot[m], b[m] * rinv);
+  out(ct->slot[kRedSlots], 0.0);
 }
 
 }  // namespace ostc
