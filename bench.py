@@ -49,18 +49,12 @@ METRIC = "Mcell-iter/s (flux+SST+chem+DPLUR), %HBM peak; surrogate vs plain chem
 # Re-measured whenever the kernel changes; a stage without an entry reports
 # null.
 MEASURED_TRAFFIC = {
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "dplur_sweep"): 2304.5e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "dplur_chem"): 4276.7e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "dplur_dq0"): 4582.7e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "source"): 1061.4e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_i"): 3578.1e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_j"): 4034.7e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_k"): 3071.3e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "update"): 1767.5e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "properties"): 730.5e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "dplur_sweep"): 514.4e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "dplur_chem"): 1195.2e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "dplur_dq0"): 1257.6e6,
     ("h2air_mixing_layer_fr_epi_dplur", "source"): 144.8e6,
     ("h2air_mixing_layer_fr_epi_dplur", "flux_i"): 671.2e6,
     ("h2air_mixing_layer_fr_epi_dplur", "flux_j"): 838.4e6,
@@ -204,26 +198,23 @@ def alg_bytes_per_cell(p, esize: int) -> dict:
     # factors and pivots read)
     if fac:
         # the chemistry after the fluxes with dq0: rho, T, Y, J, dq, dt,
-        # spectral radii 3, [J_t 2] -> dq0, the block's factors + packed pivots
-        put("dplur_dq0", 2 + ns + 1 + nv + 1 + 3 + (2 if rans else 0) + nv, na * na, npw)
+        # spectral radii 3, [J_t 2] -> dq0, the reduced block's factors (6x6
+        # and 6x2) + packed pivots
+        put("dplur_dq0", 2 + ns + 1 + nv + 1 + 3 + (2 if rans else 0) + nv, 48, npw)
     elif epi:
         put("dplur_dq0", nv + 1 + 3 + (2 if rans else 0) + nv, 2 * na * na, npw)
     else:
         put("dplur_dq0", nv + 1 + 3 + (2 if rans else 0) + nv, njac)
-    # one sweep: din, sv, u,v,w,|V|, (air p, rho | mixture T, gamma), metric 9,
-    # spectral radii 3, dt, dq0, [J_t 2] -> dout.  With EPI the species rows'
-    # block solve is its own kernel (dplur_chem): the sweep reads the flow and
-    # turbulence rows of dq0 and leaves the species rows' sums in dout, which
-    # dplur_chem reads back with dt, the species rows of dq0, the LU factors
-    # and pivots (and the spectral radii 3 when a species takes part in no
-    # reaction: its block row is the diagonal), and overwrites with the
-    # solution.
+    # one sweep, air: din, sv, u,v,w,|V|, p, rho, metric 9, spectral radii 3,
+    # dt, dq0, [J_t 2] -> dout; a mixture reads the total enthalpy and the
+    # pressure increment in place of |V|, T and gamma and writes the next
+    # sweep's pressure increment (T and gamma read for it), and with EPI it
+    # reads the block's factors and pivots
     sweep = nv + nsc + 4 + 2 + 9 + 3 + 1 + nv + (2 if rans else 0) + nv
     if epi:
-        put("dplur_sweep", sweep - ns)
-        put("dplur_chem", 2 * ns + 1 + ns + (3 if na < ns else 0), na * na, npw)
+        put("dplur_sweep", sweep + 2, 48 if fac else na * na, npw)
     else:
-        put("dplur_sweep", sweep, ns if chem else 0)
+        put("dplur_sweep", sweep + (2 if ns else 0), ns if chem else 0)
     put("dplur_sweep_first", sweep)   # reads dq in place of dq0 and writes dq0 in place of reading it
     # update: cv, dq, dt, J [T: the Newton start] -> cv, bv 6, sv, |V|
     put("update", nv + nv + 2 + (1 if ns else 0) + nv + 6 + nsc + 1)
@@ -349,7 +340,7 @@ def time_leg(case, steps: int, warmup: int, stage_steps: int):
                 # per iteration = zones x repetitions (DPLUR sweeps)
                 per_it = cnt_s[i] / stage_steps
                 reps = 1
-                if n in ("dplur_sweep", "dplur_chem"):
+                if n == "dplur_sweep":
                     reps = p.dplur_inner_step - (1 if any(x == "dplur_sweep_first" and cnt_s[j] for j, x in
                                                           enumerate(names)) and n == "dplur_sweep" else 0)
                 byts = alg[n] * cells * reps / per_it

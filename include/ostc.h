@@ -359,8 +359,9 @@ int ostc_zone_counters(ostc_zone *zone, long long out[4], int reset, void *strea
  * source kernel also forms the local time step (nothing the flux stages
  * write enters it), and in non-reacting zones the first DPLUR sweep forms
  * dq0 from dq as it loads it.  In EPI zones under DPLUR on the 9-species
- * kernels (at most 20 reactions) the finite-rate source follows the fluxes
- * in one kernel with dq0 and the chemistry block's factors: the species
+ * kernels (mechanisms whose element conservation fixes at least one reacting
+ * species, and others of at most 20 reactions) the finite-rate source follows
+ * the fluxes in one kernel with dq0 and the chemistry block's factors: the species
  * source is added to the flux residual (the reference adds the fluxes to
  * it; the sum can differ in its last bit), and the EPI Jacobian is not
  * stored (OSTC_F_CHEM_JAC then holds the block's factors).  inner faces of block b are

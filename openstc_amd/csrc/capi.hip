@@ -133,6 +133,7 @@ struct ostc_zone {
   int planes[OSTC_F_COUNT] = {};
   int fsize[OSTC_F_COUNT] = {};  // element size per field
   int *piv = nullptr;
+  void *imp = nullptr;  // ZoneView::imp
   unsigned long long *counters = nullptr;
   int *lf_count = nullptr;
   int64_t *lf_idx = nullptr;
@@ -187,6 +188,7 @@ ZoneView<R> make_view(ostc_zone *z) {
   v.dqk = P(OSTC_F_DQK);
   v.spectr = P(OSTC_F_SPECTR);
   v.dt = P(OSTC_F_DT);
+  v.imp = static_cast<R *>(z->imp);
   v.chem_jac = static_cast<double *>(z->ptr[OSTC_F_CHEM_JAC]);
   v.chem_lu = v.chem_jac;  // factors overwrite the Jacobian (it is not needed afterwards)
   v.chem_piv = z->piv;
@@ -659,6 +661,10 @@ int ostc_zone_create(ostc_ctx *ctx, const ostc_zone_desc *d, ostc_zone **out) {
   }
   if (e == hipSuccess) e = hipMalloc(&z->counters, 4 * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(z->counters, 0, 4 * sizeof(unsigned long long));
+  if (e == hipSuccess && ns > 0 && dplur) {
+    e = hipMalloc(&z->imp, (size_t)z->plane * 3 * z->esize);
+    if (e == hipSuccess) e = hipMemset(z->imp, 0, (size_t)z->plane * 3 * z->esize);
+  }
   if (e == hipSuccess) e = hipMalloc(&z->d_inflow, OSTC_MAX_BCDATA * sizeof(ostc_inflow));
   {
     // limit_flow repair list, sized for every interior cell
@@ -689,6 +695,7 @@ int ostc_zone_destroy(ostc_zone *z) {
   if (z->counters) (void)hipFree(z->counters);
   if (z->d_inflow) (void)hipFree(z->d_inflow);
   if (z->lf_count) (void)hipFree(z->lf_count);
+  if (z->imp) (void)hipFree(z->imp);
   if (z->lf_idx) (void)hipFree(z->lf_idx);
   if (z->lf_vals) (void)hipFree(z->lf_vals);
   delete z;

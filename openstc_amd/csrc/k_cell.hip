@@ -211,47 +211,6 @@ __global__ __launch_bounds__(256) void k_local_dt(ZoneView<R> z, const ostc_para
                            NT > 0 ? z.mut[id] : (R)0);
 }
 
-// The chemistry block of DPLUR, (diag I - dt J), in the space of the species
-// that react.  A species that takes part in no reaction (N2 of H2-air, the
-// inert species appended to smaller mechanisms) has a zero row and column in
-// J: a factorisation of the whole block never picks its row as a pivot (its
-// column entries are zero), its L and U entries stay zero and its U diagonal
-// stays diag, every update it enters subtracts an exact zero, and the solve
-// gives it b / diag.  So k_dq0 factors only the NA x NA block of the NA
-// species that react (ChemF64::act, in their order) and the sweeps solve that
-// block: the same values as the whole 9 x 9 factors (the sign of a zero
-// aside), with NA^2 doubles per cell instead of 81.  NA == NS takes the whole
-// block in the species' own order (the 20-species bucket, whose appended
-// inert species stay in it as zero rows and columns).  Pivots are kept as
-// positions in the block, four bits each (eight bits above 16 species),
-// packed into 32-bit planes of chem_piv.
-template <int NA>
-struct PivPack {
-  static constexpr int bits = NA > 16 ? 8 : 4, per = 32 / bits, words = (NA + per - 1) / per;
-};
-template <int NA>
-__device__ __forceinline__ void piv_pack(const int *piv, unsigned *w) {
-  using PP = PivPack<NA>;
-#pragma unroll
-  for (int q = 0; q < PP::words; ++q) w[q] = 0;
-#pragma unroll
-  for (int r = 0; r < NA; ++r) w[r / PP::per] |= (unsigned)piv[r] << (PP::bits * (r % PP::per));
-}
-template <int NA>
-__device__ __forceinline__ void piv_unpack(const unsigned *w, int *piv) {
-  using PP = PivPack<NA>;
-#pragma unroll
-  for (int r = 0; r < NA; ++r) piv[r] = (int)((w[r / PP::per] >> (PP::bits * (r % PP::per))) & ((1u << PP::bits) - 1));
-}
-// the r-th species of the block
-template <int NS, int NA>
-__device__ __forceinline__ int block_species(const ChemF64 *ct, int r) {
-  if constexpr (NA == NS)
-    return r;
-  else
-    return ct->act[r];
-}
-
 // The DPLUR chemistry block of one cell, (diag I - dt J) with diag = 1 + dt *
 // (sum of the spectral radii), formed from its whole EPI Jacobian a (NS x NS,
 // row-major) in place and factored as a whole (pivots as row indices).
@@ -690,398 +649,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   for (int m = 0; m < kRedSlots; ++m) z.dq0[(5 + ct->slot[m]) * P + id] = (R)b[m];
   const int64_t q = (5 + ct->slot[kRedSlots]) * P + id;
   z.dq0[q] = (R)((double)z.dq[q] * inv_diag);
-}
-
-// Diagonal solve and write of one cell after a DPLUR sweep has gathered its
-// off-diagonal sum acc (src/DPLURHPP.cuh:193-249); EPI_for_dqk
-// (src/FiniteRateChem.cu:255-284) with the LU factors from k_dq0.  FIRST
-// (non-reacting zones): the cell's dq0 comes in dq0v[0..NV) and is stored for
-// the later sweeps; dq0v[NV], dq0v[NV+1] hold its SST Jacobian diagonal.
-template <typename R, int NS, int NT, bool CHEM, bool FIRST>
-__device__ __forceinline__ void dplur_finish(const ZoneView<R> &z, const ostc_param *__restrict__ p, int64_t id,
-                                             const R *acc, R dt, R diag, R *__restrict__ dout, const R *dq0v) {
-  static_assert(!(FIRST && CHEM && NS > 0), "the chemistry block needs k_dq0's LU factors");
-  const int64_t P = z.plane;
-  const int nflow = (CHEM && NS > 0) ? 5 : 5 + NS;
-  auto q0 = [&](int l) -> R {
-    if constexpr (FIRST) {
-      z.dq0[l * P + id] = dq0v[l];
-      return dq0v[l];
-    } else {
-      return z.dq0[l * P + id];
-    }
-  };
-  for (int l = 0; l < nflow; ++l) dout[l * P + id] = q0(l) + dt * acc[l] / diag;
-  if constexpr (CHEM && NS > 0) {
-    const int meth = p->chem_src_method;
-    const double dtd = (double)dt, dg = (double)diag;
-    if (meth == 1) {
-      // the species rows' off-diagonal sums; k_dplur_chem solves the block
-#pragma unroll
-      for (int q = 0; q < NS; ++q) dout[(5 + q) * P + id] = acc[5 + q];
-    } else if (meth == 2) {
-#pragma unroll
-      for (int q = 0; q < NS; ++q)
-        dout[(5 + q) * P + id] =
-            (R)((double)z.dq0[(5 + q) * P + id] + dtd * (double)acc[5 + q] / (dg - dtd * z.chem_jac[q * P + id]));
-    } else {
-#pragma unroll
-      for (int q = 0; q < NS; ++q) dout[(5 + q) * P + id] = z.dq0[(5 + q) * P + id] + dt * acc[5 + q] / diag;
-    }
-  }
-  if constexpr (NT > 0) {
-    if (p->turb_implicit == 1) {
-      const R tj0 = FIRST ? dq0v[5 + NS + NT] : z.turb_jac[id];
-      const R tj1 = FIRST ? dq0v[6 + NS + NT] : z.turb_jac[P + id];
-      dout[(NS + 5) * P + id] = q0(NS + 5) + dt * acc[5 + NS] / (diag - dt * tj0);
-      dout[(NS + 6) * P + id] = q0(NS + 6) + dt * acc[6 + NS] / (diag - dt * tj1);
-    } else {
-      dout[(NS + 5) * P + id] = q0(NS + 5) + dt * acc[5 + NS] / diag;
-      dout[(NS + 6) * P + id] = q0(NS + 6) + dt * acc[6 + NS] / diag;
-    }
-  }
-}
-
-// Chemistry block of one DPLUR sweep of a reacting zone with EPI
-// (EPI_for_dqk, src/FiniteRateChem.cu:255-284): the sweep kernel leaves the
-// species rows' off-diagonal sums in dout; each cell solves its block with
-// the LU factors k_dq0 kept, dout_s = dq0_s + (diag I - dt J)^-1 (dt acc_s),
-// in place.  A kernel of its own: one streaming pass over the 9x9 FP64
-// factors with every load issued at once, instead of loads that the sweep's
-// neighbour exchange would leave exposed at the end of each plane.
-template <typename R, int NS, int NA, bool TILED = false>
-__global__ __launch_bounds__(256) void k_dplur_chem(ZoneView<R> z, const ostc_param *__restrict__ p,
-                                                    R *__restrict__ dout) {
-  const auto c = cell_index(z, 0);
-  if (!c.ok) return;
-  const int64_t id = z.idx(c.i, c.j, c.k), P = z.plane;
-  const ChemF64 *ct = chem64(p);
-  const R dt = z.dt[id];
-  const double dtd = (double)dt;
-  double a[NA * NA], b[NA];
-  int piv[NA];
-  unsigned w[PivPack<NA>::words];
-#pragma unroll
-  for (int q = 0; q < NA * NA; ++q) a[q] = z.chem_lu[TILED ? lu_tiled(id, q, NA * NA) : q * P + id];
-#pragma unroll
-  for (int q = 0; q < PivPack<NA>::words; ++q) w[q] = (unsigned)z.chem_piv[q * P + id];
-  piv_unpack<NA>(w, piv);
-#pragma unroll
-  for (int r = 0; r < NA; ++r) b[r] = (double)dout[(5 + block_species<NS, NA>(ct, r)) * P + id] * dtd;
-  lu_solve_any<NA>(a, piv, b);
-#pragma unroll
-  for (int r = 0; r < NA; ++r) {
-    const int m = block_species<NS, NA>(ct, r);
-    dout[(5 + m) * P + id] = (R)((double)z.dq0[(5 + m) * P + id] + b[r]);
-  }
-  if constexpr (NA < NS) {
-    // species that react in no reaction: their block row is diag, as k_dq0
-    // formed it
-    const double dg = (double)((R)1 + dt * (z.spectr[id] + z.spectr[P + id] + z.spectr[2 * P + id]));
-    for (int m = 0; m < NS; ++m)
-      if (ct->rank[m] < 0)
-        dout[(5 + m) * P + id] = (R)((double)z.dq0[(5 + m) * P + id] + (double)dout[(5 + m) * P + id] * dtd / dg);
-  }
-}
-
-// The same with the reduced factors of k_chem_dq0_red: 48 numbers a cell
-// instead of 64.  HBM-bound: 512 B a cell instead of 640, 0.222 -> 0.185 ms on
-// a block of 1.77 M cells (4.9 TB/s).
-template <typename R>
-__global__ __launch_bounds__(256) void k_dplur_chem_red(ZoneView<R> z, const ostc_param *__restrict__ p,
-                                                        R *__restrict__ dout) {
-  constexpr int K = kRedKept;
-  const auto c = cell_index(z, 0);
-  if (!c.ok) return;
-  const int64_t id = z.idx(c.i, c.j, c.k), P = z.plane;
-  const ChemRed *ct = chem_red(p);
-  double a[K * K], cc[K * kRedDep], b[kRedSlots];
-  int piv[K];
-#pragma unroll
-  for (int q = 0; q < K * K; ++q) a[q] = z.chem_lu[lu_tiled(id, q, kRedFactors)];
-#pragma unroll
-  for (int q = 0; q < K * kRedDep; ++q) cc[q] = z.chem_lu[lu_tiled(id, K * K + q, kRedFactors)];
-  const unsigned w = (unsigned)z.chem_piv[id];
-#pragma unroll
-  for (int q = 0; q < K; ++q) piv[q] = (int)(w >> (4 * q) & 15u);
-  const R dt = z.dt[id];
-  const double dtd = (double)dt;
-  const double inv_diag = 1.0 / (double)((R)1 + dt * (z.spectr[id] + z.spectr[P + id] + z.spectr[2 * P + id]));
-#pragma unroll
-  for (int m = 0; m < kRedSlots; ++m) b[m] = (double)dout[(5 + ct->slot[m]) * P + id] * dtd;
-  chem_red_solve(ct, a, cc, piv, inv_diag, b);
-#pragma unroll
-  for (int m = 0; m < kRedSlots; ++m) {
-    const int64_t q = (5 + ct->slot[m]) * P + id;
-    dout[q] = (R)((double)z.dq0[q] + b[m]);
-  }
-  const int64_t q = (5 + ct->slot[kRedSlots]) * P + id;
-  dout[q] = (R)((double)z.dq0[q] + (double)dout[q] * dtd * inv_diag);
-}
-
-// Per-cell inputs of the convective-Jacobian products of one DPLUR sweep
-// (the neighbour part of src/DPLURHPP.cuh:127-191), loaded once per cell.
-template <typename R, int NS, int NT>
-struct JdCell {
-  static constexpr int NV = 5 + NS + NT;
-  R d[NV];
-  R sv[NS + NT];
-  R u, v, w, e, h, b2, bb;
-  R dt, diag, tj0, tj1;  // first sweep only: the cell's dq0 scaling
-};
-
-// compute_DQ_0's diagonal scaling without a chemistry block
-// (src/DPLURHPP.cuh:13-76, SST rows src/SST.cu:196-204): d = dq / diag, the
-// same operations k_dq0 performs.  The first sweep of a non-reacting zone
-// applies it to every dq it loads instead of reading a stored dq0, and keeps
-// dt, diag and the SST Jacobian diagonal for the cell's own diagonal solve.
-template <typename R, int NS, int NT>
-__device__ __forceinline__ void dq0_scale(const ZoneView<R> &z, const ostc_param *__restrict__ p, int64_t q,
-                                          JdCell<R, NS, NT> &c) {
-  const int64_t P = z.plane;
-  c.dt = z.dt[q];
-  c.diag = (R)1 + c.dt * (z.spectr[q] + z.spectr[P + q] + z.spectr[2 * P + q]);
-  c.tj0 = c.tj1 = 0;
-#pragma unroll
-  for (int l = 0; l < 5 + NS; ++l) c.d[l] = c.d[l] / c.diag;
-  if constexpr (NT > 0) {
-    if (p->turb_implicit == 1) {
-      c.tj0 = z.turb_jac[q];
-      c.tj1 = z.turb_jac[P + q];
-      c.d[NS + 5] = c.d[NS + 5] / (c.diag - c.dt * c.tj0);
-      c.d[NS + 6] = c.d[NS + 6] / (c.diag - c.dt * c.tj1);
-    } else {
-      c.d[NS + 5] = c.d[NS + 5] / c.diag;
-      c.d[NS + 6] = c.d[NS + 6] / c.diag;
-    }
-  }
-}
-
-// FIRST: din is the right-hand side dq, scaled to dq0 on load
-template <typename R, int NS, int NT, bool FIRST>
-__device__ __forceinline__ void jd_load(const ZoneView<R> &z, const ostc_param *__restrict__ p,
-                                        const R *__restrict__ din, int64_t q, JdCell<R, NS, NT> &c) {
-  constexpr int NV = 5 + NS + NT;
-  const int64_t P = z.plane;
-#pragma unroll
-  for (int l = 0; l < NV; ++l) c.d[l] = din[l * P + q];
-  if constexpr (FIRST) dq0_scale<R, NS, NT>(z, p, q, c);
-#pragma unroll
-  for (int l = 0; l < NS + NT; ++l) c.sv[l] = z.sv[l * P + q];
-  c.u = z.bv[P + q];
-  c.v = z.bv[2 * P + q];
-  c.w = z.bv[3 * P + q];
-  const R vel = z.vel[q];
-  c.e = (R)0.5 * vel * vel;
-  R gamma = (R)kGammaAir, b3 = 0, b4 = 0;
-  if constexpr (NS > 0) {
-    R hk[NS];
-    const R t = z.bv[5 * P + q];
-    enthalpy<R>(t, hk, p, NS);
-    gamma = z.gamma[q];
-    R h = 0;
-#pragma unroll
-    for (int l = 0; l < NS; ++l) {
-      if constexpr (sizeof(R) == 4)
-        b3 += t * r_over_mw<R>(p, l) * c.d[5 + l];
-      else
-        b3 += (R)kRu * t / (R)p->mw[l] * c.d[5 + l];
-      b4 += hk[l] * c.d[5 + l];
-      h += c.sv[l] * hk[l];
-    }
-    b3 *= gamma;
-    b4 *= gamma - (R)1;
-    c.h = h + c.e;
-  } else {
-    c.h = gamma / (gamma - (R)1) * z.bv[4 * P + q] / z.bv[q] + c.e;
-  }
-  c.bb = b3 - b4;
-  c.b2 = (gamma - (R)1) * (c.e * c.d[0] - c.u * c.d[1] - c.v * c.d[2] - c.w * c.d[3] + c.d[4]);
-}
-
-// Contribution of cell q, seen as a neighbour across direction `dir`:
-// w * (A_dir(q) dq(q) + pm_sr dq(q)); out = 0.5 * (JD + sr*d) (sign +1, the
-// minus-side neighbour) or 0.5 * (JD - sr*d) (sign -1, the plus-side one).
-template <typename R, int NS, int NT>
-__device__ __forceinline__ void jd_dir(const ZoneView<R> &z, int64_t q, int dir, const JdCell<R, NS, NT> &c,
-                                       R sr, R *plus, R *minus) {
-  constexpr int NV = 5 + NS + NT;
-  const int64_t P = z.plane;
-  const R xi_x = z.metric[(dir * 3) * P + q], xi_y = z.metric[(dir * 3 + 1) * P + q],
-          xi_z = z.metric[(dir * 3 + 2) * P + q];
-  const R U = xi_x * c.u + xi_y * c.v + xi_z * c.w;
-  const R b1 = xi_x * c.d[1] + xi_y * c.d[2] + xi_z * c.d[3] - U * c.d[0];
-  R jd[NV];
-  jd[0] = b1 + U * c.d[0];
-  jd[1] = c.u * b1 + xi_x * c.b2 + U * c.d[1] + xi_x * c.bb;
-  jd[2] = c.v * b1 + xi_y * c.b2 + U * c.d[2] + xi_y * c.bb;
-  jd[3] = c.w * b1 + xi_z * c.b2 + U * c.d[3] + xi_z * c.bb;
-  jd[4] = c.h * b1 + U * c.b2 + U * c.d[4] + U * c.bb;
-#pragma unroll
-  for (int l = 0; l < NS + NT; ++l) jd[5 + l] = U * c.d[5 + l] + c.sv[l] * b1;
-#pragma unroll
-  for (int l = 0; l < NV; ++l) {
-    if (plus) plus[l] = (R)0.5 * (jd[l] + sr * c.d[l]);
-    if (minus) minus[l] = (R)0.5 * (jd[l] - sr * c.d[l]);
-  }
-}
-
-// DPLUR_inner_iteration (src/DPLURHPP.cuh:127-249): one Jacobi sweep din ->
-// dout.  A workgroup owns a 64 x 4 (i, j) tile and marches through a chunk of
-// k planes: each cell's Jacobian products are formed once per direction and
-// handed to its neighbours -- along i by lane shuffles inside the wave (one
-// wave = one i row), along j through LDS, along k in registers from the
-// previous plane.  Tile-edge neighbours outside the tile: the rows above and
-// below by the edge rows themselves (whole-wave loads); the cells left and
-// right of every row by 2*TJ lanes of an inner row's wave in one pass, handed
-// over through LDS (single-lane halo loads per row would double the tile's vector
-// memory instructions, which bound this kernel).  Off-diagonal sums are
-// accumulated in the reference's order (i-, j-, k-, i+, j+, k+).  FIRST
-// (first sweep of a non-reacting zone): din is the right-hand side dq, scaled
-// to dq0 as it is loaded, and each cell's dq0 is stored for the later sweeps
-// (no separate dq0 pass).
-template <typename R, int NS, int NT, bool CHEM, int TJ, bool FIRST>
-__global__ __launch_bounds__(64 * TJ) void k_dplur(ZoneView<R> z, const ostc_param *__restrict__ p,
-                                               const R *__restrict__ din, R *__restrict__ dout, int kc) {
-  constexpr int NV = 5 + NS + NT;
-  __shared__ R sj[2][TJ][NV][64];  // [plus/minus][row][var][lane]
-  __shared__ R si[2][TJ][NV];      // [left P_i / right M_i][row][var]
-  const int tx = threadIdx.x, ty = threadIdx.y;
-  const uint3 bk = xcd_block();
-  const int i = (int)bk.x * 64 + tx, j = (int)bk.y * TJ + ty;
-  const int k0 = (int)bk.z * kc, k1 = min(k0 + kc, z.mz);
-  const bool ok = i < z.mx && j < z.my;
-  const int ii = min(i, z.mx - 1), jj = min(j, z.my - 1);  // clamped (loads of idle lanes stay in bounds)
-  const int64_t P = z.plane;
-  const int64_t sk = (int64_t)z.nx * z.ny;
-  const R *sr = z.spectr;
-  JdCell<R, NS, NT> c;
-  R pk[NV], acc[NV], accp[NV];
-  R dq0p[FIRST ? NV + 2 : 1];  // FIRST: dq0 (+ SST diagonal) of the cell below, finished with the next plane
-  R dtp = 0, diagp = 1;
-  // P_k of the plane below the chunk
-  if (k0 > 0) {
-    const int64_t q = z.idx(ii, jj, k0 - 1);
-    jd_load<R, NS, NT, FIRST>(z, p, din, q, c);
-    jd_dir<R, NS, NT>(z, q, 2, c, sr[2 * P + q], pk, nullptr);
-  }
-  for (int k = k0; k < k1; ++k) {
-    const int64_t id = z.idx(ii, jj, k);
-    jd_load<R, NS, NT, FIRST>(z, p, din, id, c);
-    R mk[NV], pnext[NV];
-    jd_dir<R, NS, NT>(z, id, 2, c, sr[2 * P + id], pnext, mk);
-    // finish the cell below: its plus-side k neighbour is this cell
-    if (k > k0) {
-#pragma unroll
-      for (int l = 0; l < NV; ++l) accp[l] -= mk[l];
-      if (ok) dplur_finish<R, NS, NT, CHEM, FIRST>(z, p, id - sk, accp, dtp, diagp, dout, dq0p);
-    }
-    // minus-side terms in the reference order: i-, j-, k-
-    R pi[NV], mi[NV];
-    jd_dir<R, NS, NT>(z, id, 0, c, sr[id], pi, mi);
-    R pj[NV], mj[NV];
-    jd_dir<R, NS, NT>(z, id, 1, c, sr[P + id], pj, mj);
-    __syncthreads();  // previous plane's j exchange is consumed
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      sj[0][ty][l][tx] = pj[l];
-      sj[1][ty][l][tx] = mj[l];
-    }
-    // i: neighbours' P_i / M_i from the adjacent lanes
-    R ip[NV], im[NV];
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      ip[l] = __shfl_up(pi[l], 1);
-      im[l] = __shfl_down(mi[l], 1);
-    }
-    if (ty == (TJ > 2 ? 1 : 0) && tx < 2 * TJ) {
-      // lane 2r: the cell left of row r's segment (its P_i); lane 2r+1: the
-      // cell right of it (its M_i).  An inner row does this (rows 0 and TJ-1
-      // also evaluate the rows outside the tile), so that no wave carries
-      // more than two cells' loads per plane.
-      const int r = tx >> 1, side = tx & 1;
-      const int ih = side ? (int)bk.x * 64 + 64 : (int)bk.x * 64 - 1;
-      const int jr = min((int)bk.y * TJ + r, z.my - 1);
-      if (ih >= 0 && ih < z.mx) {
-        const int64_t q = z.idx(ih, jr, k);
-        JdCell<R, NS, NT> e;
-        R hp[NV], hm[NV];
-        jd_load<R, NS, NT, FIRST>(z, p, din, q, e);
-        jd_dir<R, NS, NT>(z, q, 0, e, sr[q], hp, hm);
-#pragma unroll
-        for (int l = 0; l < NV; ++l) si[side][r][l] = side ? hm[l] : hp[l];
-      }
-    }
-    // j: rows at the tile edge evaluate the neighbour row themselves
-    R jp[NV], jm[NV];
-    if (ty == 0 && j > 0) {
-      const int64_t q = z.idx(ii, j - 1, k);
-      JdCell<R, NS, NT> e;
-      jd_load<R, NS, NT, FIRST>(z, p, din, q, e);
-      jd_dir<R, NS, NT>(z, q, 1, e, sr[P + q], jp, nullptr);
-    }
-    if (ty == TJ - 1 && j + 1 < z.my) {
-      const int64_t q = z.idx(ii, j + 1, k);
-      JdCell<R, NS, NT> e;
-      jd_load<R, NS, NT, FIRST>(z, p, din, q, e);
-      jd_dir<R, NS, NT>(z, q, 1, e, sr[P + q], nullptr, jm);
-    }
-    __syncthreads();
-    if (tx == 0 && i > 0 && i - 1 < z.mx)
-#pragma unroll
-      for (int l = 0; l < NV; ++l) ip[l] = si[0][ty][l];
-    if (tx == 63 && i + 1 < z.mx)
-#pragma unroll
-      for (int l = 0; l < NV; ++l) im[l] = si[1][ty][l];
-    if (ty > 0)
-#pragma unroll
-      for (int l = 0; l < NV; ++l) jp[l] = sj[0][ty - 1][l][tx];
-    if (ty < TJ - 1)
-#pragma unroll
-      for (int l = 0; l < NV; ++l) jm[l] = sj[1][ty + 1][l][tx];
-    const bool hi = i > 0, hj = j > 0, hk = k > 0;
-    const bool lo_i = i + 1 < z.mx, lo_j = j + 1 < z.my;
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      R a = 0;
-      if (hi) a += ip[l];
-      if (hj) a += jp[l];
-      if (hk) a += pk[l];
-      if (lo_i) a -= im[l];
-      if (lo_j) a -= jm[l];
-      acc[l] = a;
-    }
-    // this plane's plus-side k term arrives with the next plane
-#pragma unroll
-    for (int l = 0; l < NV; ++l) {
-      accp[l] = acc[l];
-      pk[l] = pnext[l];
-    }
-    if constexpr (FIRST) {
-      dtp = c.dt;
-      diagp = c.diag;
-#pragma unroll
-      for (int l = 0; l < NV; ++l) dq0p[l] = c.d[l];
-      dq0p[NV] = c.tj0;
-      dq0p[NV + 1] = c.tj1;
-    } else {
-      dtp = z.dt[id];
-      diagp = (R)1 + dtp * (sr[id] + sr[P + id] + sr[2 * P + id]);
-    }
-  }
-  // last plane of the chunk: plus-side k neighbour from the plane above
-  if (k1 > k0) {
-    const int kl = k1 - 1;
-    if (k1 < z.mz) {
-      const int64_t q = z.idx(ii, jj, k1);
-      jd_load<R, NS, NT, FIRST>(z, p, din, q, c);
-      R mk[NV];
-      jd_dir<R, NS, NT>(z, q, 2, c, sr[2 * P + q], nullptr, mk);
-#pragma unroll
-      for (int l = 0; l < NV; ++l) accp[l] -= mk[l];
-    }
-    if (ok) dplur_finish<R, NS, NT, CHEM, FIRST>(z, p, z.idx(ii, jj, kl), accp, dtp, diagp, dout, dq0p);
-  }
 }
 
 // ------------------------------------------------------------------ update
@@ -1546,92 +1113,6 @@ __global__ __launch_bounds__(256) void k_wall_dist(ZoneView<R> z, const double *
 
 // ------------------------------------------------------------------ launchers
 
-// Workgroups of a DPLUR sweep kernel resident on the whole current device at
-// once (registers and LDS decide it), cached per device.
-template <typename R, int NS, int NT, bool CHEM, int TJ, bool FIRST>
-int dplur_resident() {
-  static int cached[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cached[dev] > 0) return cached[dev];
-  int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_dplur<R, NS, NT, CHEM, TJ, FIRST>, 64 * TJ, 0) !=
-          hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 0;
-  cached[dev] = per_cu * cus;
-  return cached[dev];
-}
-
-// Planes per k chunk of a DPLUR sweep over `tiles` (i, j) tiles.  The chunks
-// run in rounds of `resident` workgroups and a round lasts one chunk's march,
-// so the sweep takes about rounds x planes-per-chunk plane steps: the count
-// minimising that is taken (ties: fewer chunks, fewer boundary planes to
-// reload), with at least 4 planes per chunk.  resident <= 0 (unknown) falls
-// back to about 1024 workgroups.
-inline int dplur_chunk_planes(int tiles, int mz, int resident) {
-  const int nmax = std::max(1, (mz + 3) / 4);
-  if (resident <= 0) {
-    const int n = std::max(1, std::min((1024 + tiles - 1) / tiles, nmax));
-    return (mz + n - 1) / n;
-  }
-  int best = mz;
-  long long best_cost = -1;
-  for (int n = 1; n <= nmax; ++n) {
-    const int kc = (mz + n - 1) / n;
-    const long long chunks = (mz + kc - 1) / kc;
-    const long long rounds = ((long long)tiles * chunks + resident - 1) / resident;
-    const long long cost = rounds * kc;
-    if (best_cost < 0 || cost < best_cost) {
-      best_cost = cost;
-      best = kc;
-    }
-  }
-  return best;
-}
-
-// species of the mechanism that react (the EPI block of DPLUR), 1..9
-#define OSTC_DISPATCH_NA(o, CALL)                                  \
-  do {                                                             \
-    switch ((o).n_act) {                                           \
-      case 1: { constexpr int NA_ = 1; CALL; } break;              \
-      case 2: { constexpr int NA_ = 2; CALL; } break;              \
-      case 3: { constexpr int NA_ = 3; CALL; } break;              \
-      case 4: { constexpr int NA_ = 4; CALL; } break;              \
-      case 5: { constexpr int NA_ = 5; CALL; } break;              \
-      case 6: { constexpr int NA_ = 6; CALL; } break;              \
-      case 7: { constexpr int NA_ = 7; CALL; } break;              \
-      case 8: { constexpr int NA_ = 8; CALL; } break;              \
-      case 9: { constexpr int NA_ = 9; CALL; } break;              \
-      default: return OSTC_ERR_ARG;                                \
-    }                                                              \
-  } while (0)
-
-#define OSTC_DISPATCH_NSNT(o, CALL)              \
-  do {                                           \
-    if ((o).ns == 0 && (o).nt == 0) {            \
-      constexpr int NS_ = 0, NT_ = 0;            \
-      CALL;                                      \
-    } else if ((o).ns == 0 && (o).nt == 2) {     \
-      constexpr int NS_ = 0, NT_ = 2;            \
-      CALL;                                      \
-    } else if ((o).ns == 9 && (o).nt == 0) {     \
-      constexpr int NS_ = 9, NT_ = 0;            \
-      CALL;                                      \
-    } else if ((o).ns == 9 && (o).nt == 2) {     \
-      constexpr int NS_ = 9, NT_ = 2;            \
-      CALL;                                      \
-    } else if ((o).ns == 20 && (o).nt == 0) {    \
-      constexpr int NS_ = 20, NT_ = 0;           \
-      CALL;                                      \
-    } else if ((o).ns == 20 && (o).nt == 2) {    \
-      constexpr int NS_ = 20, NT_ = 2;           \
-      CALL;                                      \
-    } else {                                     \
-      return OSTC_ERR_ARG;                       \
-    }                                            \
-  } while (0)
-
 static inline int last_err() { return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP; }
 
 template <typename R>
@@ -1733,10 +1214,9 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
     }
     return last_err();
   }
-  // DPLUR: dq -> dq0; sweeps ping-pong dq0 -> dqk -> dq -> dqk ...  Without
-  // a chemistry block dq0 is a diagonal scaling, which the first sweep applies
-  // to the dq it loads (and stores dq0 for the later sweeps): no dq0 pass.
-  const bool fuse_dq0 = !chem && o.dplur_steps > 0;
+  // DPLUR: dq -> dq0, then the sweeps.  In air dq0 is a diagonal scaling of
+  // dq, which the sweeps apply to what they load: no dq0 pass.
+  const bool fuse_dq0 = o.ns == 0 && o.dplur_steps > 0;
   if (!fuse_dq0) {
     prof_mark(P_DQ0, st, true);
     if (chem) {
@@ -1772,63 +1252,11 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
     prof_mark(P_DQ0, st, false);
     if (last_err()) return OSTC_ERR_HIP;
   }
-  // k-marching sweeps: (64 x 4) tiles, k split into chunks sized from the
-  // resident capacity of the kernel that runs most sweeps (or so that about
-  // o.dplur_wg workgroups are in flight, when set); at least 4 planes per chunk
-  constexpr int tj = 4;
-  const int tiles = ((z.mx + 63) / 64) * ((z.my + tj - 1) / tj);
-  int kc;
-  if (o.dplur_wg > 0) {
-    const int nkc = std::max(1, std::min((o.dplur_wg + tiles - 1) / tiles, (z.mz + 3) / 4));
-    kc = (z.mz + nkc - 1) / nkc;
-  } else {
-    int resident = 0;
-    if (chem)
-      OSTC_DISPATCH_NSNT(o, resident = (dplur_resident<R, NS_, NT_, true, tj, false>()));
-    else
-      OSTC_DISPATCH_NSNT(o, resident = (dplur_resident<R, NS_, NT_, false, tj, false>()));
-    kc = dplur_chunk_planes(tiles, z.mz, resident);
+  if (o.dplur_steps == 0) {
+    *result = z.dq0;
+    return OSTC_OK;
   }
-  const dim3 sgrid((unsigned)((z.mx + 63) / 64), (unsigned)((z.my + tj - 1) / tj), (unsigned)((z.mz + kc - 1) / kc));
-  const dim3 sblock(64, tj, 1);
-  R *in = fuse_dq0 ? z.dq : z.dq0, *out = z.dqk;
-  for (int s = 0; s < o.dplur_steps; ++s) {
-    const int stage = fuse_dq0 && s == 0 ? P_DPLUR_FIRST : P_DPLUR;
-    prof_mark(stage, st, true);
-    if (chem) {
-      OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_dplur<R, NS_, NT_, true, tj, false>), sgrid, sblock, 0, st, z, dp,
-                                               (const R *)in, out, kc));
-    } else if (s == 0) {
-      OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_dplur<R, NS_, NT_, false, tj, true>), sgrid, sblock, 0, st, z, dp,
-                                               (const R *)in, out, kc));
-    } else {
-      OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_dplur<R, NS_, NT_, false, tj, false>), sgrid, sblock, 0, st, z,
-                                               dp, (const R *)in, out, kc));
-    }
-    prof_mark(stage, st, false);
-    if (last_err()) return OSTC_ERR_HIP;
-    if (chem && o.chem == 1 && o.ns > 0) {
-      prof_mark(P_DPLUR_CHEM, st, true);
-      if (o.ns == 9) {
-        // factors stored by the source kernel are tiled (lu_tiled)
-        if (chem_late && o.red)
-          hipLaunchKernelGGL((k_dplur_chem_red<R>), g.grid, g.block, 0, st, z, dp, out);
-        else if (chem_late)
-          OSTC_DISPATCH_NA(o, hipLaunchKernelGGL((k_dplur_chem<R, 9, NA_, true>), g.grid, g.block, 0, st, z, dp, out));
-        else
-          OSTC_DISPATCH_NA(o, hipLaunchKernelGGL((k_dplur_chem<R, 9, NA_>), g.grid, g.block, 0, st, z, dp, out));
-      } else if (o.ns == 20)
-        hipLaunchKernelGGL((k_dplur_chem<R, 20, 20>), g.grid, g.block, 0, st, z, dp, out);
-      else
-        return OSTC_ERR_ARG;
-      prof_mark(P_DPLUR_CHEM, st, false);
-      if (last_err()) return OSTC_ERR_HIP;
-    }
-    in = out;
-    out = (out == z.dqk) ? z.dq : z.dqk;
-  }
-  *result = in;
-  return OSTC_OK;
+  return dplur_sweeps(z, dp, o, st, chem_late, false, result);
 }
 
 // check_slot >= 0: also classify every cell for limit_flow into repair-list

@@ -468,34 +468,6 @@ __global__ __launch_bounds__(256) void sweep_kernel(ZoneView<R> z, const ostc_pa
 // derivatives 0.25*(f(L+e) - f(L-e) + f(R+e) - f(R-e)) formed as
 // 0.25*(D_e f(L) + D_e f(R)), D_e f = f(+e) - f(-e).
 
-// value of lane l-1 / l+1 (DPP wave shift; the first / last lane keeps x)
-template <typename R>
-__device__ __forceinline__ R lane_prev(R x) {
-  if constexpr (sizeof(R) == 4) {
-    const int v = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false));
-  } else {
-    const long long v = __builtin_bit_cast(long long, x);
-    const int lo = (int)v, hi = (int)(v >> 32);
-    const int a = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);
-    const int b = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
-    return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)b << 32) | (unsigned)a));
-  }
-}
-template <typename R>
-__device__ __forceinline__ R lane_next(R x) {
-  if constexpr (sizeof(R) == 4) {
-    const int v = __builtin_bit_cast(int, x);
-    return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false));
-  } else {
-    const long long v = __builtin_bit_cast(long long, x);
-    const int lo = (int)v, hi = (int)(v >> 32);
-    const int a = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);
-    const int b = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
-    return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)b << 32) | (unsigned)a));
-  }
-}
-
 // what a face needs of each of its two cells
 template <typename R, int NT>
 struct FaceCell {

@@ -59,6 +59,7 @@ struct ZoneView {
   R *rho_d, *gamma, *cp;
   R *mut, *lambda_t, *turb_jac;
   R *dq, *dq0, *dqk;
+  R *imp;             // DPLUR of a mixture: total enthalpy, then two planes of pressure increments
   R *spectr, *dt;
   double *chem_jac;   // ns*ns (EPI) or ns (DA) planes
   double *chem_lu;    // ns*ns planes: LU factors of the DPLUR chemistry block
@@ -96,6 +97,46 @@ template <typename T>
 __device__ __forceinline__ T dmin(T a, T b) { return a < b ? a : b; }
 template <typename T>
 __device__ __forceinline__ T dmax(T a, T b) { return a > b ? a : b; }
+
+// An element at a 32-bit byte offset from a wave-uniform base: the load keeps
+// its base in scalar registers and one address register serves every plane.
+// A plane of 2^32 bytes cannot be reached: a zone has at least 60 of them.
+template <typename R>
+__device__ __forceinline__ R at(const R *base, unsigned off) {
+  return *reinterpret_cast<const R *>(reinterpret_cast<const char *>(base) + off);
+}
+template <typename R>
+__device__ __forceinline__ void put(R *base, unsigned off, R v) {
+  *reinterpret_cast<R *>(reinterpret_cast<char *>(base) + off) = v;
+}
+
+// value of lane l-1 / l+1 (DPP wave shift; the first / last lane keeps x)
+template <typename R>
+__device__ __forceinline__ R lane_prev(R x) {
+  if constexpr (sizeof(R) == 4) {
+    const int v = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(v, v, 0x138, 0xf, 0xf, false));
+  } else {
+    const long long v = __builtin_bit_cast(long long, x);
+    const int lo = (int)v, hi = (int)(v >> 32);
+    const int a = __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false);
+    const int b = __builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false);
+    return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)b << 32) | (unsigned)a));
+  }
+}
+template <typename R>
+__device__ __forceinline__ R lane_next(R x) {
+  if constexpr (sizeof(R) == 4) {
+    const int v = __builtin_bit_cast(int, x);
+    return __builtin_bit_cast(R, __builtin_amdgcn_update_dpp(v, v, 0x130, 0xf, 0xf, false));
+  } else {
+    const long long v = __builtin_bit_cast(long long, x);
+    const int lo = (int)v, hi = (int)(v >> 32);
+    const int a = __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false);
+    const int b = __builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false);
+    return __builtin_bit_cast(R, (long long)(((unsigned long long)(unsigned)b << 32) | (unsigned)a));
+  }
+}
 
 // Block-id remapping so that each XCD (blocks are dealt round-robin to the 8
 // XCDs) works on one contiguous slab of the domain: stencil halos between

@@ -80,6 +80,11 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
                        bool chem_late = false);
 // check_slot >= 0: also classify every cell for limit_flow into repair-list
 // slot (check_slot & 1); then call limit_flow with the same slot.  Time steps
+// k_dplur.hip: the sweeps of implicit_treatment from dq0 (mixtures) or dq
+// (air); scalars_ready: h and s of dq0 are in z.imp
+template <typename R>
+int dplur_sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool chem_late,
+                 bool scalars_ready, R **result);
 // alternate the slot.
 template <typename R>
 int update_cv_bv(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const R *dq_final, hipStream_t st,
@@ -117,3 +122,45 @@ int chem_source_batch(const ostc_param *dp, int ns, int nr, long n, const double
                       const double *y, double *omega, double *jac, hipStream_t st);
 
 }  // namespace ostc
+// species of the mechanism that react (the EPI block of DPLUR), 1..9
+#define OSTC_DISPATCH_NA(o, CALL)                                  \
+  do {                                                             \
+    switch ((o).n_act) {                                           \
+      case 1: { constexpr int NA_ = 1; CALL; } break;              \
+      case 2: { constexpr int NA_ = 2; CALL; } break;              \
+      case 3: { constexpr int NA_ = 3; CALL; } break;              \
+      case 4: { constexpr int NA_ = 4; CALL; } break;              \
+      case 5: { constexpr int NA_ = 5; CALL; } break;              \
+      case 6: { constexpr int NA_ = 6; CALL; } break;              \
+      case 7: { constexpr int NA_ = 7; CALL; } break;              \
+      case 8: { constexpr int NA_ = 8; CALL; } break;              \
+      case 9: { constexpr int NA_ = 9; CALL; } break;              \
+      default: return OSTC_ERR_ARG;                                \
+    }                                                              \
+  } while (0)
+
+#define OSTC_DISPATCH_NSNT(o, CALL)              \
+  do {                                           \
+    if ((o).ns == 0 && (o).nt == 0) {            \
+      constexpr int NS_ = 0, NT_ = 0;            \
+      CALL;                                      \
+    } else if ((o).ns == 0 && (o).nt == 2) {     \
+      constexpr int NS_ = 0, NT_ = 2;            \
+      CALL;                                      \
+    } else if ((o).ns == 9 && (o).nt == 0) {     \
+      constexpr int NS_ = 9, NT_ = 0;            \
+      CALL;                                      \
+    } else if ((o).ns == 9 && (o).nt == 2) {     \
+      constexpr int NS_ = 9, NT_ = 2;            \
+      CALL;                                      \
+    } else if ((o).ns == 20 && (o).nt == 0) {    \
+      constexpr int NS_ = 20, NT_ = 0;           \
+      CALL;                                      \
+    } else if ((o).ns == 20 && (o).nt == 2) {    \
+      constexpr int NS_ = 20, NT_ = 2;           \
+      CALL;                                      \
+    } else {                                     \
+      return OSTC_ERR_ARG;                       \
+    }                                            \
+  } while (0)
+

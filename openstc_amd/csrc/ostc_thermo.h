@@ -3,6 +3,8 @@
 // in FP32, double for chemistry and the Newton solve).
 #pragma once
 
+#include <cstddef>
+
 #include "ostc_dev.h"
 
 namespace ostc {
@@ -1187,6 +1189,47 @@ __device__ __forceinline__ void chem_red_solve(const ChemRed *__restrict__ ct, c
     for (int n = 0; n < K; ++n) v += ct->lin[d][n] * b[n];
     b[K + d] = v;
   }
+}
+
+// The chemistry block of DPLUR, (diag I - dt J), in the space of the species
+// that react.  A species that takes part in no reaction (N2 of H2-air, the
+// inert species appended to smaller mechanisms) has a zero row and column in
+// J: a factorisation of the whole block never picks its row as a pivot (its
+// column entries are zero), its L and U entries stay zero and its U diagonal
+// stays diag, every update it enters subtracts an exact zero, and the solve
+// gives it b / diag.  So k_dq0 factors only the NA x NA block of the NA
+// species that react (ChemF64::act, in their order) and the sweeps solve that
+// block: the same values as the whole 9 x 9 factors (the sign of a zero
+// aside), with NA^2 doubles per cell instead of 81.  NA == NS takes the whole
+// block in the species' own order (the 20-species bucket, whose appended
+// inert species stay in it as zero rows and columns).  Pivots are kept as
+// positions in the block, four bits each (eight bits above 16 species),
+// packed into 32-bit planes of chem_piv.
+template <int NA>
+struct PivPack {
+  static constexpr int bits = NA > 16 ? 8 : 4, per = 32 / bits, words = (NA + per - 1) / per;
+};
+template <int NA>
+__device__ __forceinline__ void piv_pack(const int *piv, unsigned *w) {
+  using PP = PivPack<NA>;
+#pragma unroll
+  for (int q = 0; q < PP::words; ++q) w[q] = 0;
+#pragma unroll
+  for (int r = 0; r < NA; ++r) w[r / PP::per] |= (unsigned)piv[r] << (PP::bits * (r % PP::per));
+}
+template <int NA>
+__device__ __forceinline__ void piv_unpack(const unsigned *w, int *piv) {
+  using PP = PivPack<NA>;
+#pragma unroll
+  for (int r = 0; r < NA; ++r) piv[r] = (int)((w[r / PP::per] >> (PP::bits * (r % PP::per))) & ((1u << PP::bits) - 1));
+}
+// the r-th species of the block
+template <int NS, int NA>
+__device__ __forceinline__ int block_species(const ChemF64 *ct, int r) {
+  if constexpr (NA == NS)
+    return r;
+  else
+    return ct->act[r];
 }
 
 // The plain point-implicit chemistry step at fixed (T, p):
