@@ -144,6 +144,8 @@ struct ostc_zone {
   ostc_bc bc{};
   bool has_bc = false;
   ostc_inflow *d_inflow = nullptr;
+  std::vector<FaceBatch> bc_plan;  // launches of the boundary program, and their device copy
+  FaceBatch *d_bc_plan = nullptr;
   ZoneView<float> vf{};
   ZoneView<double> vd{};
 };
@@ -186,9 +188,9 @@ ZoneView<R> make_view(ostc_zone *z) {
   v.dq = P(OSTC_F_DQ);
   v.dq0 = P(OSTC_F_DQ0);
   v.dqk = P(OSTC_F_DQK);
+  v.imp = static_cast<R *>(z->imp);
   v.spectr = P(OSTC_F_SPECTR);
   v.dt = P(OSTC_F_DT);
-  v.imp = static_cast<R *>(z->imp);
   v.chem_jac = static_cast<double *>(z->ptr[OSTC_F_CHEM_JAC]);
   v.chem_lu = v.chem_jac;  // factors overwrite the Jacobian (it is not needed afterwards)
   v.chem_piv = z->piv;
@@ -659,13 +661,14 @@ int ostc_zone_create(ostc_ctx *ctx, const ostc_zone_desc *d, ostc_zone **out) {
     e = hipMalloc(&z->piv, (size_t)z->plane * ns * sizeof(int));
     if (e == hipSuccess) e = hipMemset(z->piv, 0, (size_t)z->plane * ns * sizeof(int));
   }
-  if (e == hipSuccess) e = hipMalloc(&z->counters, 4 * sizeof(unsigned long long));
-  if (e == hipSuccess) e = hipMemset(z->counters, 0, 4 * sizeof(unsigned long long));
   if (e == hipSuccess && ns > 0 && dplur) {
     e = hipMalloc(&z->imp, (size_t)z->plane * 3 * z->esize);
     if (e == hipSuccess) e = hipMemset(z->imp, 0, (size_t)z->plane * 3 * z->esize);
   }
+  if (e == hipSuccess) e = hipMalloc(&z->counters, 4 * sizeof(unsigned long long));
+  if (e == hipSuccess) e = hipMemset(z->counters, 0, 4 * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMalloc(&z->d_inflow, OSTC_MAX_BCDATA * sizeof(ostc_inflow));
+  if (e == hipSuccess) e = hipMalloc(&z->d_bc_plan, OSTC_MAX_FACE * sizeof(FaceBatch));
   {
     // limit_flow repair list, sized for every interior cell
     const size_t ncell = (size_t)d->mx * d->my * d->mz;
@@ -692,10 +695,11 @@ int ostc_zone_destroy(ostc_zone *z) {
   for (int f = 0; f < OSTC_F_COUNT; ++f)
     if (z->ptr[f]) (void)hipFree(z->ptr[f]);
   if (z->piv) (void)hipFree(z->piv);
+  if (z->imp) (void)hipFree(z->imp);
   if (z->counters) (void)hipFree(z->counters);
   if (z->d_inflow) (void)hipFree(z->d_inflow);
+  if (z->d_bc_plan) (void)hipFree(z->d_bc_plan);
   if (z->lf_count) (void)hipFree(z->lf_count);
-  if (z->imp) (void)hipFree(z->imp);
   if (z->lf_idx) (void)hipFree(z->lf_idx);
   if (z->lf_vals) (void)hipFree(z->lf_vals);
   delete z;
@@ -819,6 +823,8 @@ int ostc_zone_set_bc(ostc_zone *z, const ostc_bc *bc) {
       return fail(OSTC_ERR_ARG, "bad BC slot");
     if (b.kind != 2 && b.kind != 3 && b.kind != 5 && b.kind != 6) return fail(OSTC_ERR_ARG, "unknown BC kind");
   }
+  std::vector<FaceBatch> plan;
+  if (int r = plan_bc(*bc, g, plan)) return fail(r, "boundary program");
   z->bc = *bc;
   if (z->ctx->pad) {
     // inflow scalars [Y_0..Y_ns-1, k, omega] -> the padded layout
@@ -831,6 +837,9 @@ int ostc_zone_set_bc(ostc_zone *z, const ostc_bc *bc) {
     }
   }
   z->has_bc = true;
+  z->bc_plan.swap(plan);
+  if (!z->bc_plan.empty())
+    HIP_TRY(hipMemcpy(z->d_bc_plan, z->bc_plan.data(), z->bc_plan.size() * sizeof(FaceBatch), hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(z->d_inflow, z->bc.inflow, sizeof(z->bc.inflow), hipMemcpyHostToDevice));
   return OSTC_OK;
 }
@@ -916,8 +925,8 @@ int ostc_limit_flow(ostc_ctx *c, ostc_zone *z, void *s) {
 int ostc_apply_bc(ostc_ctx *c, ostc_zone *z, void *s) {
   if (!c || !z) return fail(OSTC_ERR_ARG, "null argument");
   if (!z->has_bc) return OSTC_OK;
-  return ZONE_CALL(z, apply_bc(z->vf, c->dev, c->opts, z->bc, z->d_inflow, S(s)),
-                   apply_bc(z->vd, c->dev, c->opts, z->bc, z->d_inflow, S(s)));
+  return ZONE_CALL(z, apply_bc(z->vf, c->dev, c->opts, z->bc_plan, z->d_bc_plan, z->d_inflow, S(s)),
+                   apply_bc(z->vd, c->dev, c->opts, z->bc_plan, z->d_bc_plan, z->d_inflow, S(s)));
 }
 
 int ostc_inner_halo(ostc_ctx *c, ostc_zone **zones, int blk, const ostc_inner_face *f, void *s) {

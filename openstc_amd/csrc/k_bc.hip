@@ -1,6 +1,6 @@
 // Boundary conditions (src/BoundCond.cuh:45-412) and the on-device inner-face
-// halo exchange (src/DataCommunication.cuh:27-98).  Each face is one launch
-// over its face points and layers, one thread per (point, layer).
+// halo exchange (src/DataCommunication.cuh:27-98): one thread per (face point,
+// layer), faces that touch no common point in one launch.
 #include <algorithm>
 
 #include "ostc_kernels.h"
@@ -10,33 +10,23 @@ namespace ostc {
 
 namespace {
 
-struct FaceLaunch {
-  int rs[3], re[3];
-  int face, direction;
-  int g0;  // first layer a launch handles: 0 = the face point, 1 = the first ghost layer
-};
-
 // Thread -> (face point, layer g): g = 0 is the face point itself, 1..ngg the
 // ghost layers outside it.  Every (point, layer) pair is independent, so the
 // layers run in parallel and each thread issues all its loads before its
 // stores.  On an i-face four adjacent lanes take the layers of one row (the
-// layers are adjacent in memory there); on j/k faces i varies fastest.
-__device__ __forceinline__ bool face_layer(const FaceLaunch &f, int ngg, int p[3], int &g) {
-  const int a = f.face == 0 ? 1 : 0, b = f.face == 2 ? 1 : 2;
-  int ia, il;
-  if (f.face == 0) {
-    il = (int)(threadIdx.x & 3);
-    ia = (int)(blockIdx.x * 16 + (threadIdx.x >> 2));
-  } else {
-    il = (int)blockIdx.z;
-    ia = (int)(blockIdx.x * 64 + threadIdx.x);
-  }
-  const int ib = (int)(blockIdx.y * blockDim.y + threadIdx.y);
+// layers are adjacent in memory there); on j/k faces i varies fastest.  id:
+// the face point's index; step: the index distance of one layer outward.
+template <typename R, int FACE>
+__device__ __forceinline__ bool face_layer(const ZoneView<R> &z, const FaceLaunch &f, uint3 blk, int64_t &id,
+                                           int64_t &step, int &g) {
+  constexpr int A = FACE == 0 ? 1 : 0, B = FACE == 2 ? 1 : 2;
+  const int il = FACE == 0 ? (int)(threadIdx.x & 3) : (int)blk.z;
+  const int ia = FACE == 0 ? (int)(blk.x * 16 + (threadIdx.x >> 2)) : (int)(blk.x * 64 + threadIdx.x);
+  const int a = f.rs[A] + ia, b = f.rs[B] + (int)(blk.y * 4 + threadIdx.y), n = f.rs[FACE];
   g = f.g0 + il;
-  p[f.face] = f.rs[f.face];
-  p[a] = f.rs[a] + ia;
-  p[b] = f.rs[b] + ib;
-  return g <= ngg && p[a] <= f.re[a] && p[b] <= f.re[b];
+  id = FACE == 0 ? z.idx(n, a, b) : (FACE == 1 ? z.idx(a, n, b) : z.idx(a, b, n));
+  step = (FACE == 0 ? (int64_t)1 : (FACE == 1 ? (int64_t)z.nx : (int64_t)z.nx * z.ny)) * f.direction;
+  return g <= z.g && a <= f.re[A] && b <= f.re[B];
 }
 
 // compute_total_energy (src/FieldOperation.cuh:15-35) of a point whose bv and
@@ -60,14 +50,13 @@ __device__ __forceinline__ R total_energy_reg(const ostc_param *__restrict__ p, 
 }
 
 // apply_outflow (src/BoundCond.cuh:127-154): ghost layer g copies the face point
-template <typename R, int NSC, bool RANS>
-__global__ __launch_bounds__(256) void k_outflow(ZoneView<R> z, FaceLaunch f) {
-  int pt[3], g;
-  if (!face_layer(f, z.g, pt, g)) return;
-  int dir[3] = {0, 0, 0};
-  dir[f.face] = f.direction;
-  const int64_t P = z.plane, id = z.idx(pt[0], pt[1], pt[2]);
-  const int64_t gi = z.idx(pt[0] + g * dir[0], pt[1] + g * dir[1], pt[2] + g * dir[2]);
+template <typename R, int NSC, bool RANS, int FACE>
+__device__ __forceinline__ void outflow_face(const ZoneView<R> &z, const FaceLaunch &f, uint3 blk) {
+  int64_t id, step;
+  int g;
+  if (!face_layer<R, FACE>(z, f, blk, id, step, g)) return;
+  const int64_t P = z.plane;
+  const int64_t gi = id + g * step;
   R bv[6], sv[NSC > 0 ? NSC : 1], mut = 0;
 #pragma unroll
   for (int l = 0; l < 6; ++l) bv[l] = z.bv[l * P + id];
@@ -82,14 +71,14 @@ __global__ __launch_bounds__(256) void k_outflow(ZoneView<R> z, FaceLaunch f) {
 }
 
 // apply_inflow (src/BoundCond.cuh:156-194): ghost layers take the inflow state
-template <typename R, int NSC, bool RANS>
-__global__ __launch_bounds__(256) void k_inflow(ZoneView<R> z, FaceLaunch f, const ostc_inflow *__restrict__ in) {
-  int pt[3], g;
-  if (!face_layer(f, z.g, pt, g)) return;
-  int dir[3] = {0, 0, 0};
-  dir[f.face] = f.direction;
+template <typename R, int NSC, bool RANS, int FACE>
+__device__ __forceinline__ void inflow_face(const ZoneView<R> &z, const FaceLaunch &f, uint3 blk,
+                                            const ostc_inflow *__restrict__ in) {
+  int64_t id, step;
+  int g;
+  if (!face_layer<R, FACE>(z, f, blk, id, step, g)) return;
   const int64_t P = z.plane;
-  const int64_t gi = z.idx(pt[0] + g * dir[0], pt[1] + g * dir[1], pt[2] + g * dir[2]);
+  const int64_t gi = id + g * step;
   z.bv[gi] = (R)in->density;
   z.bv[P + gi] = (R)in->u;
   z.bv[2 * P + gi] = (R)in->v;
@@ -104,21 +93,20 @@ __global__ __launch_bounds__(256) void k_inflow(ZoneView<R> z, FaceLaunch f, con
 // apply_symmetry (src/BoundCond.cuh:45-125): layer 0 = the face point (the
 // interior neighbour's state with its normal velocity removed), layer g = the
 // mirror of interior point -g with the normal velocity reversed
-template <typename R, int NSC, bool RANS>
-__global__ __launch_bounds__(256) void k_symmetry(ZoneView<R> z, FaceLaunch f) {
-  int pt[3], g;
-  if (!face_layer(f, z.g, pt, g)) return;
-  int dir[3] = {0, 0, 0};
-  dir[f.face] = f.direction;
-  const int64_t P = z.plane, id = z.idx(pt[0], pt[1], pt[2]);
-  R kx = z.metric[(f.face * 3) * P + id], ky = z.metric[(f.face * 3 + 1) * P + id],
-    kz = z.metric[(f.face * 3 + 2) * P + id];
+template <typename R, int NSC, bool RANS, int FACE>
+__device__ __forceinline__ void symmetry_face(const ZoneView<R> &z, const FaceLaunch &f, uint3 blk) {
+  int64_t id, step;
+  int g;
+  if (!face_layer<R, FACE>(z, f, blk, id, step, g)) return;
+  const int64_t P = z.plane;
+  R kx = z.metric[(FACE * 3) * P + id], ky = z.metric[(FACE * 3 + 1) * P + id],
+    kz = z.metric[(FACE * 3 + 2) * P + id];
   const R km = sqrt(kx * kx + ky * ky + kz * kz);
   kx /= km;
   ky /= km;
   kz /= km;
   if (g == 0) {
-    const int64_t in = z.idx(pt[0] - dir[0], pt[1] - dir[1], pt[2] - dir[2]);
+    const int64_t in = id - step;
     const R u1 = z.bv[P + in], v1 = z.bv[2 * P + in], w1 = z.bv[3 * P + in];
     const R rho = z.bv[in], pr = z.bv[4 * P + in], tt = z.bv[5 * P + in], e1 = z.cv[4 * P + in];
     R sv[NSC > 0 ? NSC : 1];
@@ -144,8 +132,8 @@ __global__ __launch_bounds__(256) void k_symmetry(ZoneView<R> z, FaceLaunch f) {
     for (int l = 0; l < NSC; ++l) z.cv[(5 + l) * P + id] = rho * sv[l];
     return;
   }
-  const int64_t gi = z.idx(pt[0] + g * dir[0], pt[1] + g * dir[1], pt[2] + g * dir[2]);
-  const int64_t si = z.idx(pt[0] - g * dir[0], pt[1] - g * dir[1], pt[2] - g * dir[2]);
+  const int64_t gi = id + g * step;
+  const int64_t si = id - g * step;
   const R rho = z.bv[si], u = z.bv[P + si], v = z.bv[2 * P + si], w = z.bv[3 * P + si];
   const R pr = z.bv[4 * P + si], tt = z.bv[5 * P + si];
   R sv[NSC > 0 ? NSC : 1], mut = 0;
@@ -170,15 +158,14 @@ __global__ __launch_bounds__(256) void k_symmetry(ZoneView<R> z, FaceLaunch f) {
 // pressure of the interior neighbour, wall or interior temperature, SST omega
 // at the wall), layer g = the reflection of interior point -g; a ghost thread
 // recomputes the wall omega it copies
-template <typename R, int NS, bool RANS>
-__global__ __launch_bounds__(256) void k_wall(ZoneView<R> z, FaceLaunch f, const ostc_param *__restrict__ p,
-                                              int isothermal, double tw_in) {
-  int pt[3], g;
-  if (!face_layer(f, z.g, pt, g)) return;
-  int dir[3] = {0, 0, 0};
-  dir[f.face] = f.direction;
-  const int64_t P = z.plane, id = z.idx(pt[0], pt[1], pt[2]);
-  const int64_t in = z.idx(pt[0] - dir[0], pt[1] - dir[1], pt[2] - dir[2]);
+template <typename R, int NS, bool RANS, int FACE>
+__device__ __forceinline__ void wall_face(const ZoneView<R> &z, const FaceLaunch &f, uint3 blk,
+                                          const ostc_param *__restrict__ p, int isothermal, double tw_in) {
+  int64_t id, step;
+  int g;
+  if (!face_layer<R, FACE>(z, f, blk, id, step, g)) return;
+  const int64_t P = z.plane;
+  const int64_t in = id - step;
   R t_wall = (R)tw_in;
   if (!isothermal) t_wall = z.bv[5 * P + in];
   const R pw = z.bv[4 * P + in];
@@ -238,8 +225,8 @@ __global__ __launch_bounds__(256) void k_wall(ZoneView<R> z, FaceLaunch f, const
     }
     return;
   }
-  const int64_t si = z.idx(pt[0] - g * dir[0], pt[1] - g * dir[1], pt[2] - g * dir[2]);
-  const int64_t gi = z.idx(pt[0] + g * dir[0], pt[1] + g * dir[1], pt[2] + g * dir[2]);
+  const int64_t si = id - g * step;
+  const int64_t gi = id + g * step;
   const R ui = z.bv[P + si], vi = z.bv[2 * P + si], wi = z.bv[3 * P + si];
   const R pi = z.bv[4 * P + si], ti = z.bv[5 * P + si];
   R ys[NS > 0 ? NS : 1];
@@ -271,6 +258,42 @@ __global__ __launch_bounds__(256) void k_wall(ZoneView<R> z, FaceLaunch f, const
     z.sv[(NS + 1) * P + gi] = om;
     z.mut[gi] = 0;
   }
+}
+
+template <typename R, int NS, int NT, int FACE>
+__device__ __forceinline__ void one_face(const ZoneView<R> &z, const BatchFace &b, uint3 blk,
+                                         const ostc_param *__restrict__ p, const ostc_inflow *__restrict__ in) {
+  constexpr int NSC = NS + NT;
+  constexpr bool RANS = NT > 0;
+  switch (b.kind) {
+    case 6: outflow_face<R, NSC, RANS, FACE>(z, b.f, blk); break;
+    case 5: inflow_face<R, NSC, RANS, FACE>(z, b.f, blk, in + b.slot); break;
+    case 3: symmetry_face<R, NSC, RANS, FACE>(z, b.f, blk); break;
+    default: wall_face<R, NS, RANS, FACE>(z, b.f, blk, p, b.isothermal, b.temperature); break;
+  }
+}
+
+// One launch over the faces of a batch.  What a launch costs is latency: the
+// batch is read from device memory (kernel arguments live in host memory),
+// the workgroup's face by the grid's z (no divisions), and the face direction
+// is a template argument (no indexed registers): the code a wave walks
+// through once, uncached, is the time.
+template <typename R, int NS, int NT>
+__global__ __launch_bounds__(256) void k_faces(ZoneView<R> z, const FaceBatch *__restrict__ batch,
+                                               const ostc_param *__restrict__ p,
+                                               const ostc_inflow *__restrict__ in) {
+  int q = 0;
+#pragma unroll
+  for (int k = 1; k < kBatchFaces; ++k) q += (int)blockIdx.z >= batch->first[k];
+  const BatchFace &b = batch->face[q];
+  if ((int)blockIdx.x >= b.gx || (int)blockIdx.y >= b.gy) return;
+  const uint3 blk = make_uint3(blockIdx.x, blockIdx.y, blockIdx.z - (unsigned)b.first);
+  if (b.f.face == 0)
+    one_face<R, NS, NT, 0>(z, b, blk, p, in);
+  else if (b.f.face == 1)
+    one_face<R, NS, NT, 1>(z, b, blk, p, in);
+  else
+    one_face<R, NS, NT, 2>(z, b, blk, p, in);
 }
 
 // update_bv_1_point (src/FieldOperation.cuh:185-215) incl. the Newton solve
@@ -391,59 +414,88 @@ __global__ __launch_bounds__(128) void k_wall_cf_qw(ZoneView<R> z, double dyn_pr
 
 }  // namespace
 
-template <typename R>
-int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const ostc_bc &bc,
-             const ostc_inflow *d_inflow, hipStream_t st) {
+namespace {
+
+// Points a face reads and writes: its ranges, and along its normal the
+// offsets lo..hi outward from the face point.
+struct FaceBox {
+  int lo[3], hi[3];
+};
+FaceBox face_box(const FaceLaunch &f, int from, int to) {
+  FaceBox b;
+  for (int q = 0; q < 3; ++q) {
+    b.lo[q] = f.rs[q];
+    b.hi[q] = f.re[q];
+  }
+  const int x = f.rs[f.face] + f.direction * from, y = f.rs[f.face] + f.direction * to;
+  b.lo[f.face] = std::min(x, y);
+  b.hi[f.face] = std::max(x, y);
+  return b;
+}
+bool meet(const FaceBox &a, const FaceBox &b) {
+  for (int q = 0; q < 3; ++q)
+    if (a.hi[q] < b.lo[q] || b.hi[q] < a.lo[q]) return false;
+  return true;
+}
+// neither face writes a point the other reads or writes
+bool independent(const FaceLaunch &a, const FaceLaunch &b, int ngg) {
+  const FaceBox wa = face_box(a, 0, ngg), wb = face_box(b, 0, ngg);
+  const FaceBox ra = face_box(a, -ngg, 0), rb = face_box(b, -ngg, 0);
+  return !meet(wa, wb) && !meet(wa, rb) && !meet(ra, wb);
+}
+
+}  // namespace
+
+int plan_bc(const ostc_bc &bc, int ngg, std::vector<FaceBatch> &batches) {
+  batches.clear();
+  if (ngg > 3) return OSTC_ERR_ARG;  // four lanes per point on i-faces
   for (int fi = 0; fi < bc.n_face; ++fi) {
     const ostc_face &bf = bc.face[fi];
-    FaceLaunch f;
-    for (int q = 0; q < 3; ++q) {
-      f.rs[q] = bf.range_start[q];
-      f.re[q] = bf.range_end[q];
+    BatchFace q{};
+    FaceLaunch &f = q.f;
+    for (int d = 0; d < 3; ++d) {
+      f.rs[d] = bf.range_start[d];
+      f.re[d] = bf.range_end[d];
     }
     f.face = bf.face;
     f.direction = bf.direction;
     f.g0 = (bf.kind == 5 || bf.kind == 6) ? 1 : 0;  // inflow/outflow write only the ghost layers
-    if (z.g > 3) return OSTC_ERR_ARG;               // four lanes per point on i-faces
+    for (int d = 0; d < 3; ++d)
+      if (d != f.face && f.re[d] < f.rs[d]) return OSTC_ERR_ARG;  // an empty face
     dim3 block;
-    const dim3 grid = face_grid(f, z.g, block);
-    const int nsc = o.ns + o.nt;
-    const bool rans = o.nt > 0;
-#define OSTC_BC_SC(KERNEL, ...)                                                              \
-  do {                                                                                       \
-    if (nsc == 0 && !rans) hipLaunchKernelGGL((KERNEL<R, 0, false>), grid, block, 0, st, __VA_ARGS__); \
-    else if (nsc == 2 && rans) hipLaunchKernelGGL((KERNEL<R, 2, true>), grid, block, 0, st, __VA_ARGS__); \
-    else if (nsc == 9 && !rans) hipLaunchKernelGGL((KERNEL<R, 9, false>), grid, block, 0, st, __VA_ARGS__); \
-    else if (nsc == 11 && rans) hipLaunchKernelGGL((KERNEL<R, 11, true>), grid, block, 0, st, __VA_ARGS__); \
-    else if (nsc == 20 && !rans) hipLaunchKernelGGL((KERNEL<R, 20, false>), grid, block, 0, st, __VA_ARGS__); \
-    else if (nsc == 22 && rans) hipLaunchKernelGGL((KERNEL<R, 22, true>), grid, block, 0, st, __VA_ARGS__); \
-    else return OSTC_ERR_ARG;                                                                \
-  } while (0)
-    switch (bf.kind) {
-      case 6: OSTC_BC_SC(k_outflow, z, f); break;
-      case 5: OSTC_BC_SC(k_inflow, z, f, d_inflow + bf.slot); break;
-      case 3: OSTC_BC_SC(k_symmetry, z, f); break;
-      case 2: {
-        const ostc_wall &w = bc.wall[bf.slot];
-        if (o.ns == 0 && !rans)
-          hipLaunchKernelGGL((k_wall<R, 0, false>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else if (o.ns == 0 && rans)
-          hipLaunchKernelGGL((k_wall<R, 0, true>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else if (o.ns == 9 && !rans)
-          hipLaunchKernelGGL((k_wall<R, 9, false>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else if (o.ns == 9 && rans)
-          hipLaunchKernelGGL((k_wall<R, 9, true>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else if (o.ns == 20 && !rans)
-          hipLaunchKernelGGL((k_wall<R, 20, false>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else if (o.ns == 20 && rans)
-          hipLaunchKernelGGL((k_wall<R, 20, true>), grid, block, 0, st, z, f, dp, w.isothermal, w.temperature);
-        else
-          return OSTC_ERR_ARG;
-        break;
-      }
-      default: return OSTC_ERR_ARG;
+    const dim3 grid = face_grid(f, ngg, block);
+    q.kind = bf.kind;
+    q.slot = bf.slot;
+    q.gx = (int)grid.x;
+    q.gy = (int)grid.y;
+    if (bf.kind == 2) {
+      q.isothermal = bc.wall[bf.slot].isothermal;
+      q.temperature = bc.wall[bf.slot].temperature;
     }
-#undef OSTC_BC_SC
+    bool joins = !batches.empty() && batches.back().n < kBatchFaces;
+    if (joins)
+      for (int k = 0; k < batches.back().n && joins; ++k) joins = independent(batches.back().face[k].f, f, ngg);
+    if (!joins) batches.emplace_back();
+    FaceBatch &b = batches.back();
+    q.first = b.gz;
+    b.first[b.n] = b.gz;
+    b.face[b.n++] = q;
+    b.gx = std::max(b.gx, q.gx);
+    b.gy = std::max(b.gy, q.gy);
+    b.gz += (int)grid.z;
+  }
+  for (auto &b : batches)
+    for (int k = b.n; k < kBatchFaces; ++k) b.first[k] = b.gz;
+  return OSTC_OK;
+}
+
+template <typename R>
+int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const std::vector<FaceBatch> &plan,
+             const FaceBatch *d_plan, const ostc_inflow *d_inflow, hipStream_t st) {
+  for (size_t q = 0; q < plan.size(); ++q) {
+    const dim3 grid((unsigned)plan[q].gx, (unsigned)plan[q].gy, (unsigned)plan[q].gz), block(64, 4, 1);
+    OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_faces<R, NS_, NT_>), grid, block, 0, st, z, d_plan + q, dp,
+                                             d_inflow));
     if (hipGetLastError() != hipSuccess) return OSTC_ERR_HIP;
   }
   return OSTC_OK;
@@ -494,10 +546,10 @@ int wall_friction_heatflux(const ZoneView<R> &z, double dyn_pressure, double *cf
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
-template int apply_bc<float>(const ZoneView<float> &, const ostc_param *, const CellOpts &, const ostc_bc &,
-                             const ostc_inflow *, hipStream_t);
-template int apply_bc<double>(const ZoneView<double> &, const ostc_param *, const CellOpts &, const ostc_bc &,
-                              const ostc_inflow *, hipStream_t);
+template int apply_bc<float>(const ZoneView<float> &, const ostc_param *, const CellOpts &,
+                             const std::vector<FaceBatch> &, const FaceBatch *, const ostc_inflow *, hipStream_t);
+template int apply_bc<double>(const ZoneView<double> &, const ostc_param *, const CellOpts &,
+                              const std::vector<FaceBatch> &, const FaceBatch *, const ostc_inflow *, hipStream_t);
 template int inner_halo<float>(const ZoneView<float> &, const ZoneView<float> &, const ostc_param *,
                                const CellOpts &, const ostc_inner_face &, hipStream_t);
 template int inner_halo<double>(const ZoneView<double> &, const ZoneView<double> &, const ostc_param *,

@@ -1,6 +1,8 @@
 // Host-side launchers of the device kernels (one translation unit each).
 #pragma once
 
+#include <vector>
+
 #include "ostc_dev.h"
 
 namespace ostc {
@@ -78,13 +80,13 @@ int local_time_step(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &
 template <typename R>
 int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, R **result,
                        bool chem_late = false);
-// check_slot >= 0: also classify every cell for limit_flow into repair-list
-// slot (check_slot & 1); then call limit_flow with the same slot.  Time steps
 // k_dplur.hip: the sweeps of implicit_treatment from dq0 (mixtures) or dq
 // (air); scalars_ready: h and s of dq0 are in z.imp
 template <typename R>
 int dplur_sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool chem_late,
                  bool scalars_ready, R **result);
+// check_slot >= 0: also classify every cell for limit_flow into repair-list
+// slot (check_slot & 1); then call limit_flow with the same slot.  Time steps
 // alternate the slot.
 template <typename R>
 int update_cv_bv(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const R *dq_final, hipStream_t st,
@@ -104,9 +106,33 @@ template <typename R>
 int wall_distance(const ZoneView<R> &z, const double *wall_xyz, int n_wall, hipStream_t st);
 
 // k_bc.hip
+// A boundary face as its kernel takes it.
+struct FaceLaunch {
+  int rs[3], re[3];
+  int face, direction;
+  int g0;  // first layer a launch handles: 0 = the face point, 1 = the first ghost layer
+};
+struct BatchFace {
+  FaceLaunch f;
+  int first, gx, gy;  // its first grid plane, and its workgroups along the two face directions
+  int kind, slot, isothermal;
+  double temperature;
+};
+// Faces of one launch: consecutive faces of the boundary program that touch
+// no common point, so that their order does not matter.  A face is a few
+// microseconds of latency whatever its size, and a block has six to ten of
+// them one after another.
+constexpr int kBatchFaces = 8;
+struct FaceBatch {
+  int n = 0, gx = 0, gy = 0, gz = 0;  // faces, launch grid
+  int first[kBatchFaces] = {};
+  BatchFace face[kBatchFaces] = {};
+};
+// the launches of a boundary program, in its order
+int plan_bc(const ostc_bc &bc, int ngg, std::vector<FaceBatch> &batches);
 template <typename R>
-int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const ostc_bc &bc,
-             const ostc_inflow *d_inflow, hipStream_t st);
+int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const std::vector<FaceBatch> &plan,
+             const FaceBatch *d_plan, const ostc_inflow *d_inflow, hipStream_t st);
 template <typename R>
 int inner_halo(const ZoneView<R> &z, const ZoneView<R> &t, const ostc_param *dp, const CellOpts &o,
                const ostc_inner_face &f, hipStream_t st);
@@ -121,7 +147,6 @@ int chem_plain_step(const ostc_param *dp, int ns, int nr, bool red, long n, cons
 int chem_source_batch(const ostc_param *dp, int ns, int nr, long n, const double *rho, const double *t,
                       const double *y, double *omega, double *jac, hipStream_t st);
 
-}  // namespace ostc
 // species of the mechanism that react (the EPI block of DPLUR), 1..9
 #define OSTC_DISPATCH_NA(o, CALL)                                  \
   do {                                                             \
@@ -164,3 +189,4 @@ int chem_source_batch(const ostc_param *dp, int ns, int nr, long n, const double
     }                                            \
   } while (0)
 
+}  // namespace ostc
