@@ -1290,30 +1290,28 @@ ostc::SurParams sur_params(const ostc_surrogate_desc &d) {
 int sur_ensure_fallback(ostc_surrogate *s, long n) {
   if (n <= s->st.fb_cap) return OSTC_OK;
   HIP_TRY(hipDeviceSynchronize());
-  for (void *buf : {(void *)s->st.fb_list, (void *)s->st.out12}) {
-    if (!buf) continue;
+  if (s->st.rejected) {
     for (auto &q : s->owned)
-      if (q == buf) q = nullptr;
-    HIP_TRY(hipFree(buf));
+      if (q == s->st.rejected) q = nullptr;
+    HIP_TRY(hipFree(s->st.rejected));
   }
-  s->st.fb_list = nullptr;
-  s->st.out12 = nullptr;
+  s->st.rejected = nullptr;
   s->st.fb_cap = 0;
-  HIP_TRY(sur_alloc(s, &s->st.fb_list, (size_t)ostc::kFbLists * ostc::fb_list_cap(n)));
-  HIP_TRY(sur_alloc(s, &s->st.out12, (size_t)n * 12));
+  HIP_TRY(sur_alloc(s, &s->st.rejected, (size_t)n));
   s->st.fb_cap = n;
   return OSTC_OK;
 }
 
-int sur_read_stats(ostc_surrogate *s, long long stats[4], hipStream_t st) {
+int sur_read_stats(ostc_surrogate *s, long n, long long stats[4], hipStream_t st) {
   if (!stats) return OSTC_OK;
-  unsigned long long h[ostc::kFbLists * ostc::kStatStride];
-  HIP_TRY(hipMemcpyAsync(h, s->st.stats, sizeof(h), hipMemcpyDeviceToHost, st));
+  std::vector<unsigned long long> h((size_t)s->st.cus * 4);
+  HIP_TRY(hipMemcpyAsync(h.data(), s->st.stats, h.size() * sizeof(h[0]), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
-  for (int q = 0; q < 4; ++q) {
+  stats[0] = n;
+  for (int q = 1; q < 4; ++q) {
     unsigned long long v = 0;
-    for (int l = 0; l < ostc::kFbLists; ++l) v += h[l * ostc::kStatStride + q];
-    stats[q] = (long long)v;
+    for (int l = 0; l < s->st.cus; ++l) v += h[(size_t)l * 4 + q];
+    stats[q] = n > 0 ? (long long)v : 0;
   }
   return OSTC_OK;
 }
@@ -1358,8 +1356,7 @@ int ostc_surrogate_create(ostc_ctx *ctx, const ostc_surrogate_desc *desc, const 
   S.packed = pk;
   A(&S.bias, (size_t)ostc::kSurBias);
   A(&S.loss_w, 16);
-  A(&S.fb_count, (size_t)ostc::kFbLists * ostc::kFbStride);
-  A(&S.stats, (size_t)ostc::kFbLists * ostc::kStatStride);
+  A(&S.stats, (size_t)S.cus * 4);
   if (max_batch > 0) {
     const size_t B = (size_t)max_batch;
     A(&S.a0, B * 16);
@@ -1427,7 +1424,7 @@ int ostc_surrogate_step(ostc_surrogate *s, long n, const double *t, const double
   if (st) return st;
   st = ostc::sur_infer_batch(s->st, s->ctx->dev, n, t, p, y, dt, dy, nullptr, S(strm));
   if (st) return fail(st, "surrogate inference launch failed");
-  return sur_read_stats(s, stats, S(strm));
+  return sur_read_stats(s, n, stats, S(strm));
 }
 
 int ostc_surrogate_forward(ostc_surrogate *s, long n, const double *t, const double *p, const double *y,
@@ -1480,7 +1477,7 @@ int ostc_chem_zone_step(ostc_ctx *c, ostc_zone *z, ostc_surrogate *s, int mode, 
   st = fp64(z) ? ostc::sur_infer_zone(s->st, c->dev, z->vd, dy, S(strm))
                : ostc::sur_infer_zone(s->st, c->dev, z->vf, dy, S(strm));
   if (st) return fail(st, "surrogate inference launch failed");
-  return sur_read_stats(s, stats, S(strm));
+  return sur_read_stats(s, n, stats, S(strm));
 }
 
 }  // extern "C"

@@ -43,9 +43,8 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kNs = 9;
-constexpr int kWaves = 12;             // waves per workgroup of the fused kernel (3 per SIMD)
-constexpr int kTiles = 4;              // 16-cell slabs per wave pass (64 cells)
-constexpr int kStageLd = 9;            // padded LDS staging row: 8 values per cell
+constexpr int kWaves = 12;    // waves per workgroup of the inference kernel (3 per SIMD)
+constexpr int kStageLd = 13;  // LDS staging row of a cell: 6 dwords of BF16 features, then 12 outputs (padded)
 
 // LDS hand-off between the lanes of one wave
 __device__ __forceinline__ void wave_sync() {
@@ -173,13 +172,13 @@ struct ZoneSrc {
 // BoxCox_0.1(Y_k) = (Y^0.1 - 1)/0.1, ln dt (logarithms and powers through the
 // hardware log2/exp2).
 constexpr float kLn2 = 0.6931471805599453f;
-__device__ __forceinline__ void features(const SurParams &s, double T, double P, const double *Y, double DT,
+__device__ __forceinline__ void features(const SurParams &s, double T, double P, const float *Y, double DT,
                                          float *f) {
   f[0] = 1000.0f / (float)T;
   f[1] = __builtin_amdgcn_logf((float)P * kInvAtm) * kLn2;
 #pragma unroll
   for (int k = 0; k < kNs; ++k) {
-    const float y = fmaxf((float)Y[k], 0.0f);
+    const float y = fmaxf(Y[k], 0.0f);
     f[2 + k] = (fast_exp2(kBoxCox * __builtin_amdgcn_logf(y)) - 1.0f) * kInvBoxCox;
   }
   f[11] = __builtin_amdgcn_logf((float)DT) * kLn2;
@@ -196,12 +195,10 @@ struct TrainOut {
 };
 
 struct InferOut {
-  float *out12;                  // [n][12] standardised outputs (forward -> decode)
   double *dy;                    // [n][9]
-  int *fb_count;                 // sub-list lengths (stride kFbStride)
-  long *fb_list;                 // sub-lists of fallback cells, fb_cap apart
-  long fb_cap;                   // capacity of one sub-list
-  unsigned long long *stats;     // statistics rows (stride kStatStride)
+  unsigned *rejected;            // [n]: each workgroup's rejected cells (less its first cell), from its first cell on
+  unsigned long long *stats;     // [stat_rows][4], a row per workgroup: its first cell, cells rejected for each reason
+  int stat_rows;
   float *raw;                    // optional [n][16] standardised outputs
 };
 
@@ -234,287 +231,298 @@ __device__ __forceinline__ int tile_l0(int mt) { return mt; }
 __device__ __forceinline__ int tile_h(int l, int mt, int kc) { return 8 + (l - 1) * 32 + mt * 4 + kc; }
 __device__ __forceinline__ int tile_out(int kc) { return 104 + kc; }
 
-template <typename Src, bool TRAIN, int ACT>
-__global__ __launch_bounds__(kWaves * 64) void k_sur_forward(SurParams s, Src src, const bf16x8 *__restrict__ wpk,
+// The whole network for CELLS cells per wave pass (features one lane per cell,
+// then the layers for 16 * TILES cells at a time), and for inference the
+// decoding, the checks and the store of the accepted changes, one lane per
+// cell again.  A pass keeps its cells' mass fractions and the input check in
+// registers from the features to the checks, so the states are read once and
+// the outputs never leave the chip; the rejected cells go to the workgroup's
+// list, placed by one LDS atomic a pass.  Bound by the activations' vector
+// instructions (512 a cell: 5 plain, 2 transcendental, which issue at half
+// rate): 84 % of the issue slots at 1 M cells.  The layers run on 32 cells at
+// a time so that the matrix results of one 32-unit chunk can be activated
+// while the next chunk's products run.  With a decode kernel behind it and the
+// outputs in memory between them the step took 443 us at 1.5 M cells, now
+// 340.  TRAIN and small batches take 16 cells per wave: 4 096 samples are then
+// 64 workgroups instead of 6 (loss gradients 309 -> 222 us).
+template <typename Src, bool TRAIN, int ACT, int CELLS, int TILES, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void k_sur_forward(SurParams s, Src src, const bf16x8 *__restrict__ wpk,
                                                             const float *__restrict__ bias, TrainOut tr,
                                                             InferOut io) {
+  static_assert(CELLS % (16 * TILES) == 0 && CELLS <= 64, "cells per pass");
   __shared__ bf16x8 sW[kSurTiles * 64];
   __shared__ __attribute__((aligned(16))) float sB[kSurBias];
-  __shared__ float sStage[kWaves][64 * kStageLd];
-  static_assert(kWaves * 64 >= kFbLists, "workgroup 0 clears every sub-list counter");
-  if constexpr (!TRAIN) {
-    // clear the fallback sub-list counters and statistics rows that the
-    // decode kernel (next on the stream) appends to
-    if (blockIdx.x == 0 && threadIdx.x < kFbLists && io.fb_count) {
-      io.fb_count[threadIdx.x * kFbStride] = 0;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) io.stats[threadIdx.x * kStatStride + r] = 0;
-    }
-  }
-  for (int q = threadIdx.x; q < kSurTiles * 64; q += blockDim.x) sW[q] = wpk[q];
-  for (int q = threadIdx.x; q < kSurBias; q += blockDim.x) sB[q] = bias[q];
+  __shared__ float sStage[WAVES][CELLS * kStageLd];
+  __shared__ unsigned rejected[4];  // cells in all and by reason
+  if (threadIdx.x < 4) rejected[threadIdx.x] = 0;
+  // nine loads in flight a thread
+  static_assert(kSurTiles % WAVES == 0, "whole rounds of weight tiles");
+#pragma unroll 9
+  for (int q = 0; q < kSurTiles / WAVES; ++q)
+    sW[q * WAVES * 64 + threadIdx.x] = wpk[q * WAVES * 64 + threadIdx.x];
+  for (int q = threadIdx.x; q < kSurBias; q += WAVES * 64) sB[q] = bias[q];
   __syncthreads();
 
   const int wave = threadIdx.x >> 6, ln = threadIdx.x & 63, g = ln >> 4, cn = ln & 15;
   const long n = src.n;
-  const long stride = (long)gridDim.x * kWaves * 64;
-  for (long base = ((long)blockIdx.x * kWaves + wave) * 64; base < n; base += stride) {
+  // each wave takes an equal run of parts (16 * TILES cells), up to CELLS
+  // cells a pass: with whole passes dealt out in turn the last round would
+  // leave most waves idle
+  constexpr int kPart = 16 * TILES;
+  const long parts = (n + kPart - 1) / kPart;
+  const int waves = (int)gridDim.x * WAVES, w = (int)blockIdx.x * WAVES + wave;
+  const long each = parts / waves;
+  const int more = (int)(parts - each * waves);  // waves with one part more, spread over the workgroups
+  auto first_cell = [&](int v) {
+    return (each * v + (int)((unsigned)v * (unsigned)more / (unsigned)waves)) * kPart;
+  };
+  const long wg0 = first_cell((int)blockIdx.x * WAVES), end = min(n, first_cell(w + 1));
+  for (long base = first_cell(w); base < end; base += CELLS) {
+    const int live = (int)min((long)CELLS, end - base);  // cells of this pass
     float *stg = sStage[wave];
-    // ---- features, one lane per cell, staged through LDS in two halves
-    // (rows hold 8 values: features 0..7, then 8..11)
-    float f[kSurIn];
-    {
+    // ---- features, one lane per cell, as BF16 pairs in the cell's staging row
+    float yf[kNs];
+    bool in_box = false;
+    if (ln < CELLS) {
       const long c = base + ln;
+      float f[kSurIn];
 #pragma unroll
       for (int q = 0; q < kSurIn; ++q) f[q] = 0.0f;
-      if (c < n) {
+      if (ln < live) {
         double T, P, DT, Y[kNs];
         src.load(c, T, P, Y, DT);
-        features(s, T, P, Y, DT, f);
+        in_box = sur_in_box(s, T, P, DT);
+#pragma unroll
+        for (int k = 0; k < kNs; ++k) {
+          yf[k] = (float)Y[k];
+          in_box = in_box && Y[k] >= -s.y_tol;
+        }
+        features(s, T, P, yf, DT, f);
       }
+      unsigned *row = reinterpret_cast<unsigned *>(stg + ln * kStageLd);
 #pragma unroll
-      for (int q = 0; q < 8; ++q) stg[ln * kStageLd + q] = f[q];
+      for (int q = 0; q < kSurIn / 2; ++q) row[q] = pack_bf16(f[2 * q], f[2 * q + 1]);
     }
     wave_sync();
-    // ---- layer 0 operand: slots 8g..8g+7 of the 32-slot chunk = features
-    // (g = 0: features 0..7, g = 1: features 8..11 then zeros, g > 1: zeros)
-    bf16x8 b0[kTiles];
+#pragma unroll 1
+    for (int part = 0; part * kPart < live; ++part) {
+      const long base_p = base + (long)part * kPart;
+      // the weight tiles are read again in every part (kept over the loop they
+      // would spill)
+      asm volatile("" ::: "memory");
+      // ---- layer 0 operands: slots 8g..8g+7 of the 32-slot chunk = features
+      // (g = 0: features 0..7, g = 1: features 8..11 then zeros, g > 1: zeros)
+      bf16x8 b0[TILES];
 #pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      const float *row = stg + (16 * t + cn) * kStageLd;
-      uint4 u;
-      u.x = g == 0 ? pack_bf16(row[0], row[1]) : 0u;
-      u.y = g == 0 ? pack_bf16(row[2], row[3]) : 0u;
-      u.z = g == 0 ? pack_bf16(row[4], row[5]) : 0u;
-      u.w = g == 0 ? pack_bf16(row[6], row[7]) : 0u;
-      b0[t] = __builtin_bit_cast(bf16x8, u);
-    }
-    wave_sync();
-#pragma unroll
-    for (int q = 0; q < kSurIn - 8; ++q) stg[ln * kStageLd + q] = f[8 + q];
-    wave_sync();
-#pragma unroll
-    for (int t = 0; t < kTiles; ++t) {
-      const float *row = stg + (16 * t + cn) * kStageLd;
-      if (g == 1) {
+      for (int t = 0; t < TILES; ++t) {
+        const unsigned *row = reinterpret_cast<const unsigned *>(stg + (part * kPart + 16 * t + cn) * kStageLd);
         uint4 u;
-        u.x = pack_bf16(row[0], row[1]);
-        u.y = pack_bf16(row[2], row[3]);
-        u.z = 0u;
-        u.w = 0u;
+        u.x = g < 2 ? row[4 * (g & 1)] : 0u;
+        u.y = g < 2 ? row[4 * (g & 1) + 1] : 0u;
+        u.z = g == 0 ? row[2] : 0u;
+        u.w = g == 0 ? row[3] : 0u;
         b0[t] = __builtin_bit_cast(bf16x8, u);
-      }
-
-      const long c = base + 16 * t + cn;
-      if (TRAIN && c < n && g < 2) {
-        float4 *dst = reinterpret_cast<float4 *>(tr.a0 + c * 16 + 8 * g);
-        dst[0] = make_float4((float)b0[t][0], (float)b0[t][1], (float)b0[t][2], (float)b0[t][3]);
-        if (g == 0)
-          dst[1] = make_float4((float)b0[t][4], (float)b0[t][5], (float)b0[t][6], (float)b0[t][7]);
-        else
-          dst[1] = make_float4(1.0f, 0.0f, 0.0f, 0.0f);  // bias column for the weight gradient
-      }
-    }
-    // the staging rows are rewritten by the next pass (their reads above are
-    // consumed before the first MFMA)
-    __builtin_amdgcn_wave_barrier();
-
-    bf16x8 bc[4][kTiles];  // current layer input: [k chunk][slab]
-    // ---- layer 0: 12 (padded 32) -> 128; the bias enters as the MFMA's C
-#pragma unroll
-    for (int kc = 0; kc < 4; ++kc) {
-      f32x4 acc[2][kTiles];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const f32x4 bz = *reinterpret_cast<const f32x4 *>(&sB[32 * kc + 16 * h + 4 * g]);
-        const bf16x8 a = sW[tile_l0(2 * kc + h) * 64 + ln];
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t)
-          acc[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0[t], bz, 0, 0, 0);
-      }
-#pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        bc[kc][t] = act_pack<ACT>(acc[0][t], acc[1][t]);
-        if (TRAIN) save_layer(tr, 0, n, base + 16 * t + cn, 32 * kc + 4 * g, acc[0][t], acc[1][t], bc[kc][t]);
-      }
-    }
-    // ---- hidden layers 1..3: 128 -> 128
-#pragma unroll
-    for (int l = 1; l <= 3; ++l) {
-      bf16x8 bn[4][kTiles];
-      // the 32 A tiles of the layer in issue order q = (kc*4 + ki)*2 + h,
-      // each read from LDS one step ahead of its MFMAs
-      bf16x8 abuf[2];
-      abuf[0] = sW[tile_h(l, 0, 0) * 64 + ln];
-#pragma unroll
-      for (int kc = 0; kc < 4; ++kc) {
-        f32x4 acc[2][kTiles];
-        f32x4 bz[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) bz[h] = *reinterpret_cast<const f32x4 *>(&sB[128 * l + 32 * kc + 16 * h + 4 * g]);
-#pragma unroll
-        for (int ki = 0; ki < 4; ++ki)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int q = (kc * 4 + ki) * 2 + h;
-            if (q + 1 < 32) {
-              const int qn = q + 1;
-              abuf[qn & 1] = sW[tile_h(l, 2 * (qn >> 3) + (qn & 1), (qn >> 1) & 3) * 64 + ln];
-            }
-            const bf16x8 a = abuf[q & 1];
-#pragma unroll
-            for (int t = 0; t < kTiles; ++t)
-              acc[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bc[ki][t], ki == 0 ? bz[h] : acc[h][t], 0, 0, 0);
-          }
-#pragma unroll
-        for (int t = 0; t < kTiles; ++t) {
-          bn[kc][t] = act_pack<ACT>(acc[0][t], acc[1][t]);
-          if (TRAIN) save_layer(tr, l, n, base + 16 * t + cn, 32 * kc + 4 * g, acc[0][t], acc[1][t], bn[kc][t]);
+        const long c = base_p + 16 * t + cn;
+        if (TRAIN && c < n && g < 2) {
+          float4 *dst = reinterpret_cast<float4 *>(tr.a0 + c * 16 + 8 * g);
+          dst[0] = make_float4((float)b0[t][0], (float)b0[t][1], (float)b0[t][2], (float)b0[t][3]);
+          if (g == 0)
+            dst[1] = make_float4((float)b0[t][4], (float)b0[t][5], (float)b0[t][6], (float)b0[t][7]);
+          else
+            dst[1] = make_float4(1.0f, 0.0f, 0.0f, 0.0f);  // bias column for the weight gradient
         }
       }
+      // the rows are rewritten with this part's outputs below (their reads
+      // are consumed before the first MFMA)
+      __builtin_amdgcn_wave_barrier();
+      bf16x8 bc[4][TILES];  // current layer input: [k chunk][slab]
+      // ---- layer 0: 12 (padded 32) -> 128; the bias enters as the MFMA's C
 #pragma unroll
-      for (int kc = 0; kc < 4; ++kc)
+      for (int kc = 0; kc < 4; ++kc) {
+        f32x4 acc[2][TILES];
 #pragma unroll
-        for (int t = 0; t < kTiles; ++t) bc[kc][t] = bn[kc][t];
-    }
-    if (TRAIN && g == 0) {
-      // bias column (1, then zero padding) of the activations feeding layers 1..4
+        for (int h = 0; h < 2; ++h) {
+          const f32x4 bz = *reinterpret_cast<const f32x4 *>(&sB[32 * kc + 16 * h + 4 * g]);
+          const bf16x8 a = sW[tile_l0(2 * kc + h) * 64 + ln];
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        const long c = base + 16 * t + cn;
-        if (c < n)
-          for (int l = 0; l < 4; ++l) {
-            float4 *dst = reinterpret_cast<float4 *>(tr.a + ((long)l * n + c) * 144 + 128);
-            dst[0] = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
-            dst[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            dst[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            dst[3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          for (int t = 0; t < TILES; ++t)
+            acc[h][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0[t], bz, 0, 0, 0);
+        }
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+          bc[kc][t] = act_pack<ACT>(acc[0][t], acc[1][t]);
+          if (TRAIN) save_layer(tr, 0, n, base_p + 16 * t + cn, 32 * kc + 4 * g, acc[0][t], acc[1][t], bc[kc][t]);
+        }
+      }
+      // ---- hidden layers 1..3: 128 -> 128
+#pragma unroll
+      for (int l = 1; l <= 3; ++l) {
+        bf16x8 bn[4][TILES];
+        // the 32 A tiles of the layer in issue order q = (kc*4 + ki)*2 + h,
+        // each read from LDS one step ahead of its MFMAs
+        bf16x8 abuf[2];
+        abuf[0] = sW[tile_h(l, 0, 0) * 64 + ln];
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) {
+          f32x4 acc[2][TILES];
+          f32x4 bz[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            bz[h] = *reinterpret_cast<const f32x4 *>(&sB[128 * l + 32 * kc + 16 * h + 4 * g]);
+#pragma unroll
+          for (int ki = 0; ki < 4; ++ki)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int q = (kc * 4 + ki) * 2 + h;
+              if (q + 1 < 32) {
+                const int qn = q + 1;
+                abuf[qn & 1] = sW[tile_h(l, 2 * (qn >> 3) + (qn & 1), (qn >> 1) & 3) * 64 + ln];
+              }
+              const bf16x8 a = abuf[q & 1];
+#pragma unroll
+              for (int t = 0; t < TILES; ++t)
+                acc[h][t] =
+                    __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bc[ki][t], ki == 0 ? bz[h] : acc[h][t], 0, 0, 0);
+            }
+#pragma unroll
+          for (int t = 0; t < TILES; ++t) {
+            bn[kc][t] = act_pack<ACT>(acc[0][t], acc[1][t]);
+            if (TRAIN) save_layer(tr, l, n, base_p + 16 * t + cn, 32 * kc + 4 * g, acc[0][t], acc[1][t], bn[kc][t]);
           }
+        }
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+#pragma unroll
+          for (int t = 0; t < TILES; ++t) bc[kc][t] = bn[kc][t];
+      }
+      if (TRAIN && g == 0) {
+        // bias column (1, then zero padding) of the activations feeding layers 1..4
+#pragma unroll
+        for (int t = 0; t < TILES; ++t) {
+          const long c = base_p + 16 * t + cn;
+          if (c < n)
+            for (int l = 0; l < 4; ++l) {
+              float4 *dst = reinterpret_cast<float4 *>(tr.a + ((long)l * n + c) * 144 + 128);
+              dst[0] = make_float4(1.0f, 0.0f, 0.0f, 0.0f);
+              dst[1] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+              dst[2] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+              dst[3] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
+      }
+      // ---- output layer: 128 -> n_out (padded 16); lane (g, cn) holds
+      // outputs 4g..4g+3 of cell 16t+cn
+      f32x4 acc[TILES];
+      const f32x4 bo = *reinterpret_cast<const f32x4 *>(&sB[512 + 4 * g]);
+#pragma unroll
+      for (int ki = 0; ki < 4; ++ki) {
+        const bf16x8 a = sW[tile_out(ki) * 64 + ln];
+#pragma unroll
+        for (int t = 0; t < TILES; ++t)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bc[ki][t], ki == 0 ? bo : acc[t], 0, 0, 0);
+      }
+#pragma unroll
+      for (int t = 0; t < TILES; ++t) {
+        const long c = base_p + 16 * t + cn;
+        if constexpr (TRAIN) {
+          if (c < n)
+            *reinterpret_cast<float4 *>(tr.yout + c * 16 + 4 * g) =
+                make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+        } else {
+          // outputs 12..15 are padding; this part's feature rows are consumed
+          if (g < 3) {
+            float *row = stg + (part * kPart + 16 * t + cn) * kStageLd + 4 * g;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) row[q] = acc[t][q];
+          }
+          if (io.raw && c < n)
+            *reinterpret_cast<float4 *>(io.raw + c * 16 + 4 * g) =
+                g < 3 ? make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]) : make_float4(0, 0, 0, 0);
+        }
       }
     }
-    // ---- output layer: 128 -> n_out (padded 16)
-    f32x4 acc[kTiles];
-    const f32x4 bo = *reinterpret_cast<const f32x4 *>(&sB[512 + 4 * g]);
+    if constexpr (!TRAIN) {
+      // ---- decode and checks, one lane per cell
+      wave_sync();
+      const long c = base + ln;
+      int why = 0;  // 0 accepted, 1 input range, 2 output range, 3 element balance
+      if (ln < live) {
+        float o[16], dy[kNs];
 #pragma unroll
-    for (int ki = 0; ki < 4; ++ki) {
-      const bf16x8 a = sW[tile_out(ki) * 64 + ln];
+        for (int q = 0; q < 12; ++q) o[q] = stg[ln * kStageLd + q];
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t)
-        acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bc[ki][t], ki == 0 ? bo : acc[t], 0, 0, 0);
-    }
-    if (TRAIN) {
+        for (int q = 12; q < 16; ++q) o[q] = 0.0f;
+        sur_decode(s, o, dy);
+        why = in_box ? sur_check_change(s, yf, dy) : 1;
+        if (why == 0) {
 #pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        const long c = base + 16 * t + cn;
-        if (c < n)
-          *reinterpret_cast<float4 *>(tr.yout + c * 16 + 4 * g) =
-              make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+          for (int k = 0; k < kNs; ++k) io.dy[c * kNs + k] = (double)dy[k];
+        }
       }
-      continue;
-    }
-    // standardised outputs in the accumulator layout: lane (g, cn) holds
-    // outputs 4g..4g+3 of cell 16t+cn (outputs 12..15 are padding)
-    if (g < 3) {
-#pragma unroll
-      for (int t = 0; t < kTiles; ++t) {
-        const long c = base + 16 * t + cn;
-        if (c < n)
-          *reinterpret_cast<float4 *>(io.out12 + c * 12 + 4 * g) =
-              make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+      const unsigned long long lo = __ballot(why & 1), hi = __ballot(why & 2), any = lo | hi;
+      if (any) {
+        unsigned at = 0;
+        if (ln < 4)
+          at = atomicAdd(&rejected[ln],
+                         (unsigned)__popcll(ln == 0 ? any : (ln == 1 ? lo & ~hi : (ln == 2 ? hi & ~lo : lo & hi))));
+        at = __builtin_amdgcn_readfirstlane(at);
+        if (why) io.rejected[wg0 + at + __popcll(any & ((1ull << ln) - 1ull))] = (unsigned)(c - wg0);
       }
+      wave_sync();  // the rows are read before the next pass writes them
     }
+  }
+  if constexpr (!TRAIN) {
+    // the workgroup's row, and the rows without a workgroup cleared
+    __syncthreads();
+    if (threadIdx.x < 4)
+      io.stats[(long)blockIdx.x * 4 + threadIdx.x] =
+          threadIdx.x == 0 ? (unsigned long long)wg0 : (unsigned long long)rejected[threadIdx.x];
+    if (blockIdx.x == 0)
+      for (int q = gridDim.x * 4 + threadIdx.x; q < io.stat_rows * 4; q += blockDim.x) io.stats[q] = 0;
   }
 }
 
-// Decode + checks, one thread per cell: accepted cells store dY, the others
-// join the wave's fallback sub-list (one atomic per wave).
-template <typename Src>
-__global__ __launch_bounds__(256) void k_sur_decode(SurParams s, Src src, InferOut io) {
-  const long c = (long)blockIdx.x * 256 + threadIdx.x;
-  const int ln = threadIdx.x & 63;
-  int why = 0;  // 0 accepted, 1 input range, 2 output range, 3 element balance
-  if (c < src.n) {
-    float o[16];
-    const float4 *r4 = reinterpret_cast<const float4 *>(io.out12 + c * 12);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const float4 v = r4[q];
-      o[4 * q] = v.x;
-      o[4 * q + 1] = v.y;
-      o[4 * q + 2] = v.z;
-      o[4 * q + 3] = v.w;
-    }
-#pragma unroll
-    for (int q = 12; q < 16; ++q) o[q] = 0.0f;
-    double T, P, DT, Y[kNs];
-    src.load(c, T, P, Y, DT);
-    if (io.raw) {
-#pragma unroll
-      for (int q = 0; q < 16; q += 4)
-        *reinterpret_cast<float4 *>(io.raw + c * 16 + q) = make_float4(o[q], o[q + 1], o[q + 2], o[q + 3]);
-    }
-    float dy[kNs];
-    sur_decode(s, o, dy);
-    why = sur_check(s, T, P, DT, Y, dy);
-    if (why == 0) {
-#pragma unroll
-      for (int k = 0; k < kNs; ++k) io.dy[c * kNs + k] = (double)dy[k];
-    }
-  }
-  const int list = (int)((c >> 6) % kFbLists);
-  const unsigned long long fail = __ballot(why != 0);
-  if (fail) {
-    const int first = __ffsll((long long)fail) - 1;
-    int at = 0;
-    if (ln == first) at = atomicAdd(io.fb_count + list * kFbStride, __popcll(fail));
-    at = __shfl(at, first);
-    if (why != 0) io.fb_list[list * io.fb_cap + at + __popcll(fail & ((1ull << ln) - 1ull))] = c;
-  }
-  if (io.stats) {
-    unsigned long long *row = io.stats + list * kStatStride;
-    const unsigned long long valid = __ballot(c < src.n);
-    if (ln == 0) atomicAdd(&row[0], (unsigned long long)__popcll(valid));
-#pragma unroll
-    for (int r = 1; r <= 3; ++r) {
-      const unsigned long long m = __ballot(why == r);
-      if (m && ln == 0) atomicAdd(&row[r], (unsigned long long)__popcll(m));
-    }
-  }
+// The chemistry's tables into the L2, a line per lane: behind a batch's states
+// none of them is left there, and the reaction loop would fetch its records
+// one after the other (the launch at 1 M cells: 42 -> 32 us).
+__device__ __forceinline__ int touch_tables(const ostc_param *__restrict__ p, int ln) {
+  int x = 0;
+  auto lines = [&](const void *t, int bytes) {
+    for (int o = ln * 128; o < bytes; o += 64 * 128)
+      x ^= *reinterpret_cast<const int *>(static_cast<const char *>(t) + o);
+  };
+  lines(chem_red(p), (int)sizeof(ChemRed));
+  lines(chem64(p), (int)sizeof(ChemF64));
+  return x;
 }
 
-// Plain point-implicit step on the fallback sub-lists (grid-stride over their
-// total, which lives on the device; entry q is found by a binary search over
-// the sub-list offsets).
+// Plain point-implicit step on the cells that the checks rejected, 64 a wave:
+// the wave takes its share of one workgroup's list (written on the same XCD:
+// the grid is `per` times the forward's, a multiple of 8 where it is large).
+// What it costs is one step's latency as long as no SIMD has two waves of it,
+// so the lists are kept dense: rejected cells come in clusters, and with a
+// fixed run of cells for each wave some had to go round twice (1 M states, 1.8
+// % rejected: 48 us).
 template <typename Src, bool RED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_sur_fallback(
-    const ostc_param *__restrict__ p, Src src,
-                                                      const int *__restrict__ count, const long *__restrict__ list,
-                                                      long cap, double *__restrict__ dyo) {
-  __shared__ int pre[kFbLists + 1];
+    const ostc_param *__restrict__ p, Src src, const unsigned *__restrict__ rejected,
+    const unsigned long long *__restrict__ stats, int wgs, int per, double *__restrict__ dyo) {
   __shared__ ConcGibbs tab_mem[RED ? kRedEntries * 64 : 1];
-  for (int l = threadIdx.x; l < kFbLists; l += blockDim.x) pre[l + 1] = count[l * kFbStride];
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    pre[0] = 0;
-    for (int l = 1; l <= kFbLists; ++l) pre[l] += pre[l - 1];
+  const int wg = (int)blockIdx.x % wgs, ln = threadIdx.x;
+  const unsigned long long *row = stats + (long)wg * 4;
+  const int m = (int)(row[1] + row[2] + row[3]), first = (int)blockIdx.x / wgs * 64;
+  if (first >= m) return;
+  if constexpr (RED) {
+    const int warm = touch_tables(p, ln);
+    asm volatile("" ::"v"(warm));
   }
-  __syncthreads();
-  const int m = pre[kFbLists];
-  for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < m; q += gridDim.x * blockDim.x) {
-    int lo = 0, hi = kFbLists;  // pre[lo] <= q < pre[hi]
-    while (hi - lo > 1) {
-      const int mid = (lo + hi) >> 1;
-      if (pre[mid] <= q)
-        lo = mid;
-      else
-        hi = mid;
-    }
-    const long c = list[lo * cap + (q - pre[lo])];
+  const long wg0 = (long)row[0];
+  for (int q = first + ln; q < m; q += per * 64) {
+    const long c = wg0 + rejected[wg0 + q];
     double T, P, DT, Y[kNs];
     src.load(c, T, P, Y, DT);
     if constexpr (RED) {
-      plain_chem_step_red(p, T, P, Y, DT, tab_mem + threadIdx.x, 64,
-                          [&](int k, double v) { dyo[c * kNs + k] = v; });
+      plain_chem_step_red(p, T, P, Y, DT, tab_mem + ln, 64, [&](int k, double v) { dyo[c * kNs + k] = v; });
     } else {
       double dy[kNs];
       plain_chem_step<kNs>(p, T, P, Y, DT, dy);
@@ -724,43 +732,38 @@ int sur_pack(const SurState &st, hipStream_t s) {
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
-static unsigned forward_grid(long n, int cus) {
-  const long wgs = (n + kWaves * 64 - 1) / (kWaves * 64);
-  return (unsigned)std::max<long>(1, std::min<long>(wgs, cus));
-}
-
-template <typename Src, bool TRAIN>
-static void launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
+template <typename Src, bool TRAIN, int CELLS, int TILES, int WAVES>
+static int launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
                            hipStream_t s) {
-  const dim3 grid(forward_grid(src.n, st.cus)), block(kWaves * 64);
+  const long wgs = (src.n + WAVES * CELLS - 1) / (WAVES * CELLS);
+  const dim3 grid((unsigned)std::max<long>(1, std::min<long>(wgs, st.cus))), block(WAVES * 64);
   const bf16x8 *wpk = reinterpret_cast<const bf16x8 *>(st.packed);
   if (st.params.act == OSTC_SUR_HSWISH)
-    hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_HSWISH>), grid, block, 0, s, st.params, src, wpk,
-                       st.bias, tr, io);
+    hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_HSWISH, CELLS, TILES, WAVES>), grid, block, 0, s,
+                       st.params, src, wpk, st.bias, tr, io);
   else
-    hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_GELU>), grid, block, 0, s, st.params, src, wpk, st.bias,
-                       tr, io);
+    hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_GELU, CELLS, TILES, WAVES>), grid, block, 0, s,
+                       st.params, src, wpk, st.bias, tr, io);
+  return (int)grid.x;
 }
 
 template <typename Src>
 static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, double *dy, float *raw,
                       hipStream_t s) {
   TrainOut tr{};
-  InferOut io{st.out12, dy, st.fb_count, st.fb_list, fb_list_cap(st.fb_cap), st.stats, raw};
-  launch_forward<Src, false>(st, src, tr, io, s);
-  hipLaunchKernelGGL(k_sur_decode<Src>, dim3((unsigned)((src.n + 255) / 256)), dim3(256), 0, s, st.params, src,
-                     io);
-  // one wave per workgroup (the kernel's launch bound), enough of them to
-  // spread a typical fallback list over every CU; the kernel strides over
-  // the device-side count
-  const long fb_blocks = std::min<long>((src.n + 63) / 64, 16L * st.cus);
-  const dim3 fb_grid((unsigned)std::max<long>(1, fb_blocks));
+  InferOut io{dy, st.rejected, st.stats, st.cus, raw};
+  // batches that 64-cell passes would leave on part of the CUs: 16 cells a wave
+  const int wgs = src.n < 64L * kWaves * st.cus / 2 ? launch_forward<Src, false, 16, 1, 4>(st, src, tr, io, s)
+                                                    : launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
+  // one wave per 64 cells of a workgroup, at most two a SIMD
+  const int per = (int)std::min<long>(8, (src.n / wgs + 32 * kWaves + 63) / 64);
+  const dim3 fb_grid((unsigned)(wgs * per));
   if (st.red)
-    hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.fb_count, st.fb_list,
-                       fb_list_cap(st.fb_cap), dy);
+    hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.stats,
+                       wgs, per, dy);
   else
-    hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.fb_count, st.fb_list,
-                       fb_list_cap(st.fb_cap), dy);
+    hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.stats,
+                       wgs, per, dy);
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
@@ -801,7 +804,7 @@ int sur_gradients(const SurState &st, long nb, const double *t, const double *p,
   BatchSrc src{t, p, y, dt, idx, nb};
   TrainOut tr{st.a0, st.z, st.a, st.yout};
   InferOut io{};
-  launch_forward<BatchSrc, true>(st, src, tr, io, s);
+  launch_forward<BatchSrc, true, 16, 1, 4>(st, src, tr, io, s);
   const unsigned lblocks = (unsigned)((nb * 16 + 255) / 256);
   hipLaunchKernelGGL(k_sur_loss, dim3(lblocks), dim3(256), 0, s, st.yout, target, idx, st.loss_w,
                      st.params.n_out, nb, st.g5, st.loss_part);

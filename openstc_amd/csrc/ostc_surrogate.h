@@ -23,19 +23,6 @@ constexpr float kInvAtm = (float)(1.0 / 101325.0);
 constexpr float kBoxCox = 0.1f;
 constexpr float kInvBoxCox = 10.0f;
 constexpr float kAdamB1 = 0.9f, kAdamB2 = 0.999f, kAdamEps = 1e-8f;
-// The fallback list is split into kFbLists sub-lists, each with its own
-// counter (and row of statistics) 128 bytes apart: wave w of the decode kernel
-// appends to sub-list w % kFbLists, so the list atomics spread over many
-// memory channels instead of serialising on one address.
-constexpr int kFbLists = 64;
-constexpr int kFbStride = 32;    // ints between two sub-list counters
-constexpr int kStatStride = 16;  // u64 between two statistics rows
-// capacity of one sub-list for n cells (its waves times 64 cells)
-__host__ __device__ inline long fb_list_cap(long n) {
-  const long waves = (n + 63) / 64;
-  return (waves + kFbLists - 1) / kFbLists * 64;
-}
-
 // parameter layout: per layer W[out][in] row-major, then b[out]
 __host__ __device__ inline int sur_in_dim(int l) { return l == 0 ? kSurIn : kSurHidden; }
 __host__ __device__ inline int sur_out_dim(int l, int n_out) { return l == 4 ? n_out : kSurHidden; }
@@ -68,11 +55,9 @@ struct SurState {
   void *packed = nullptr;  // kSurTiles * 64 lanes * 8 BF16
   float *bias = nullptr;   // kSurBias
   float *loss_w = nullptr; // 16
-  int *fb_count = nullptr;                 // [kFbLists * kFbStride]
-  long *fb_list = nullptr;                 // [kFbLists][fb_list_cap(fb_cap)]
-  float *out12 = nullptr;  // [fb_cap][12] standardised outputs of the forward kernel
-  long fb_cap = 0;
-  unsigned long long *stats = nullptr;  // [kFbLists * kStatStride], 4 used per row
+  unsigned *rejected = nullptr;  // [fb_cap] cells the checks rejected, by forward workgroup
+  long fb_cap = 0;               // cells `rejected` is sized for
+  unsigned long long *stats = nullptr;  // [cus][4], a row per workgroup: its first cell, cells rejected by reason
   // training buffers (max_batch rows)
   float *a0 = nullptr, *z = nullptr, *a = nullptr, *yout = nullptr, *g5 = nullptr;
   float *gbuf[2] = {nullptr, nullptr};
@@ -93,21 +78,28 @@ __device__ __forceinline__ void sur_decode(const SurParams &s, const float *o, f
   }
 }
 
-// 0 = accepted; 1 = input outside the trained box; 2 = Y+dY outside
+// 0 = accepted; 1 = input outside the trained box (T, P, dt here, and every
+// Y_k >= -y_tol); 2 = Y+dY outside
 // [-y_tol, 1+y_tol] or |dY_k| > dy_max; 3 = element balance
 // sum_k a_jk dY_k/W_k violated.
-__device__ __forceinline__ int sur_check(const SurParams &s, double T, double P, double DT, const double *Y,
-                                         const float *dy) {
-  bool in = (T >= s.t_min && T <= s.t_max && P >= s.p_min && P <= s.p_max && DT >= s.dt_min && DT <= s.dt_max);
-#pragma unroll
-  for (int k = 0; k < 9; ++k) in = in && (Y[k] >= -s.y_tol);
-  if (!in) return 1;
+__device__ __forceinline__ bool sur_in_box(const SurParams &s, double T, double P, double DT) {
+  return T >= s.t_min && T <= s.t_max && P >= s.p_min && P <= s.p_max && DT >= s.dt_min && DT <= s.dt_max;
+}
+// the checks of a change dy of an input inside the box; y: Y rounded to FP32
+__device__ __forceinline__ int sur_check_change(const SurParams &s, const float *y, const float *dy) {
+  // smallest and largest Y+dY and the largest |dY|; a NaN among them fails
+  // its own comparison
   bool out = true;
+  float lo = y[0] + dy[0], hi = lo, big = fabsf(dy[0]);
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    const float yn = (float)Y[k] + dy[k];
-    out = out && (yn >= -s.y_tol && yn <= 1.0f + s.y_tol) && fabsf(dy[k]) <= s.dy_max;
+    const float yn = y[k] + dy[k];
+    out = out && yn == yn;
+    lo = fminf(lo, yn);
+    hi = fmaxf(hi, yn);
+    big = fmaxf(big, fabsf(dy[k]));
   }
+  out = out && lo >= -s.y_tol && hi <= 1.0f + s.y_tol && big <= s.dy_max;
   if (!out) return 2;
   float tot = 0.0f, worst = 0.0f;
   for (int j = 0; j < s.n_elem; ++j) {
