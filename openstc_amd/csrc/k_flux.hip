@@ -11,6 +11,9 @@
 //  * j/k-sweeps: tile = 64 cells (i) x L cells along the sweep; faces are
 //    enumerated i-fastest so every wavefront reads one contiguous i-row.
 // The tile's first face is shared with the previous tile (recomputed, 1/L).
+#include <algorithm>
+#include <atomic>
+#include <cmath>
 #include <cstdlib>
 
 #include "ostc_kernels.h"
@@ -876,24 +879,64 @@ __global__ __launch_bounds__(256) void k_flux_march(ZoneView<R> z, const ostc_pa
   }
 }
 
+// Workgroups of a marching flux kernel resident on the whole current device,
+// kept per device (every thread that forms one finds the same number).
+template <typename R, int NT, int M, bool I, bool V, int A>
+static int march_resident() {
+  static std::atomic<int> kept[64] = {};
+  int dev = 0, per_cu = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (const int r = kept[dev].load(std::memory_order_relaxed)) return r;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_flux_march<R, NT, M, I, V, A>, 256, 0) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  kept[dev].store(per_cu * cus, std::memory_order_relaxed);
+  return per_cu * cus;
+}
+
+// Rows marched per wave, 1..8.  A chunk of r rows costs r steps and about two
+// more for its first rows (three are loaded besides), and the chunks run in
+// rounds of `resident` workgroups; up to two rounds they are whole, past that
+// the last one overlaps the others and counts half.  A small block takes short
+// chunks, so that every CU has some: 64x64x8 FP64 inviscid, whole iteration
+// 72 us at 8 rows, 40 at 1; 256x128x64 FP32 SST 762 us at 8, 776 at 4, 780 at
+// 11.
+static int march_rows(long long tiles, int rows, int resident) {
+  static const int fixed = [] {  // launch tuning; environment override
+    const char *e = std::getenv("OSTC_FLUX_MLEN");
+    return e ? std::max(1, std::atoi(e)) : 0;
+  }();
+  if (fixed > 0) return fixed;
+  if (resident <= 0) return std::min(8, rows);
+  int best = 1;
+  double best_cost = 0;
+  for (int r = 1; r <= std::min(8, rows); ++r) {
+    const double fill = (double)(tiles * ((rows + r - 1) / r)) / resident;
+    const double cost = (fill <= 2.0 ? std::ceil(fill) : fill + 0.5) * (r + 2);
+    if (r == 1 || cost <= best_cost) {
+      best = r;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 template <typename R, int NT>
 static int launch_march(const ZoneView<R> &z, const ostc_param *dp, bool inv, bool visc, bool first_writer,
                         hipStream_t st, bool keep_turb) {
   const int segs = (z.mx + kSegUseful - 1) / kSegUseful;
-  // rows marched per wave (launch tuning; 3 extra rows are loaded per chunk)
-  static const int mlen = [] {
-    const char *e = std::getenv("OSTC_FLUX_MLEN");
-    const int v = e ? std::atoi(e) : 8;
-    return v < 1 ? 1 : v;
-  }();
   const dim3 block(64, 4);
-#define OSTC_MARCH(M, I, V, A) \
-  hipLaunchKernelGGL((k_flux_march<R, NT, M, I, V, A>), grid, block, 0, st, z, dp, mlen)
+#define OSTC_MARCH(M, I, V, A)                                                                       \
+  do {                                                                                               \
+    const int mlen = march_rows((long long)segs * rowsX, extM, march_resident<R, NT, M, I, V, A>()); \
+    const dim3 grid((unsigned)segs, (unsigned)rowsX, (unsigned)((extM + mlen - 1) / mlen));          \
+    hipLaunchKernelGGL((k_flux_march<R, NT, M, I, V, A>), grid, block, 0, st, z, dp, mlen);          \
+  } while (0)
   for (int m = 1; m <= 2; ++m) {
     if (m == 2 && z.mz == 1) break;
     const int X = 3 - m;
     const int extX = X == 1 ? z.my : z.mz, extM = m == 1 ? z.my : z.mz;
-    const dim3 grid((unsigned)segs, (unsigned)((extX + 3) / 4), (unsigned)((extM + mlen - 1) / mlen));
+    const int rowsX = (extX + 3) / 4;
     const int acc = !(first_writer && m == 1) ? 1 : (keep_turb && NT > 0 ? 2 : 0);
     prof_mark(m == 1 ? P_FLUX_IJ : P_FLUX_K, st, true);
     if (m == 1) {
