@@ -899,7 +899,7 @@ static int march_resident() {
 // rounds of `resident` workgroups; up to two rounds they are whole, past that
 // the last one overlaps the others and counts half.  A small block takes short
 // chunks, so that every CU has some: 64x64x8 FP64 inviscid, whole iteration
-// 72 us at 8 rows, 40 at 1; 256x128x64 FP32 SST 762 us at 8, 776 at 4, 780 at
+// 72 us at 8 rows, 41 at 1; 256x128x64 FP32 SST 762 us at 8, 776 at 4, 780 at
 // 11.
 static int march_rows(long long tiles, int rows, int resident) {
   static const int fixed = [] {  // launch tuning; environment override

@@ -121,7 +121,8 @@ struct BatchFace {
 // Faces of one launch: consecutive faces of the boundary program that touch
 // no common point, so that their order does not matter.  A face is a few
 // microseconds of latency whatever its size, and a block has six to ten of
-// them one after another.
+// them one after another (mixing layer, each pass: 45 us in a launch a face,
+// 7.6 together).
 constexpr int kBatchFaces = 8;
 struct FaceBatch {
   int n = 0, gx = 0, gy = 0, gz = 0;  // faces, launch grid
