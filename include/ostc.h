@@ -148,6 +148,11 @@ int ostc_zone_upload(ostc_zone *zone, int field, const double *host, int n_plane
 int ostc_zone_download(const ostc_zone *zone, int field, double *host, int n_planes);
 /* Device pointer and element size of a field (for zero-copy callers). */
 int ostc_zone_field_ptr(const ostc_zone *zone, int field, void **dev_ptr, int *elem_size);
+/* Boundary program of the zone.  A boundary pass that is queued or captured
+ * keeps the faces, wall flags and wall temperatures it was launched with.  The
+ * inflow states are read when a pass runs: the call waits for the device
+ * before it changes them (queued passes take the old ones, a captured pass
+ * the ones set last).  On an error the zone keeps its program. */
 int ostc_zone_set_bc(ostc_zone *zone, const ostc_bc *bc);
 int ostc_sizeof_param(void);
 int ostc_sizeof_bc(void);

@@ -141,11 +141,9 @@ struct ostc_zone {
   // repair-list slot (0/1) of the next checking update in ostc_steady_step:
   // the zone alternates it itself, so callers may repeat or skip step numbers
   int lf_slot = 0;
-  ostc_bc bc{};
   bool has_bc = false;
   ostc_inflow *d_inflow = nullptr;
-  std::vector<FaceBatch> bc_plan;  // launches of the boundary program, and their device copy
-  FaceBatch *d_bc_plan = nullptr;
+  std::vector<FaceBatch> bc_plan;  // launches of the boundary program
   ZoneView<float> vf{};
   ZoneView<double> vd{};
 };
@@ -668,7 +666,6 @@ int ostc_zone_create(ostc_ctx *ctx, const ostc_zone_desc *d, ostc_zone **out) {
   if (e == hipSuccess) e = hipMalloc(&z->counters, 4 * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMemset(z->counters, 0, 4 * sizeof(unsigned long long));
   if (e == hipSuccess) e = hipMalloc(&z->d_inflow, OSTC_MAX_BCDATA * sizeof(ostc_inflow));
-  if (e == hipSuccess) e = hipMalloc(&z->d_bc_plan, OSTC_MAX_FACE * sizeof(FaceBatch));
   {
     // limit_flow repair list, sized for every interior cell
     const size_t ncell = (size_t)d->mx * d->my * d->mz;
@@ -698,7 +695,6 @@ int ostc_zone_destroy(ostc_zone *z) {
   if (z->imp) (void)hipFree(z->imp);
   if (z->counters) (void)hipFree(z->counters);
   if (z->d_inflow) (void)hipFree(z->d_inflow);
-  if (z->d_bc_plan) (void)hipFree(z->d_bc_plan);
   if (z->lf_count) (void)hipFree(z->lf_count);
   if (z->lf_idx) (void)hipFree(z->lf_idx);
   if (z->lf_vals) (void)hipFree(z->lf_vals);
@@ -825,22 +821,24 @@ int ostc_zone_set_bc(ostc_zone *z, const ostc_bc *bc) {
   }
   std::vector<FaceBatch> plan;
   if (int r = plan_bc(*bc, g, plan)) return fail(r, "boundary program");
-  z->bc = *bc;
+  ostc_bc next = *bc;
   if (z->ctx->pad) {
     // inflow scalars [Y_0..Y_ns-1, k, omega] -> the padded layout
     const int u = z->ctx->user_ns, b = z->ctx->host.n_spec, nt = z->ctx->host.n_scalar - b;
-    for (auto &in : z->bc.inflow) {
+    for (auto &in : next.inflow) {
       double sv[OSTC_MAX_SPEC + 2] = {};
       for (int l = 0; l < u; ++l) sv[l] = in.sv[l];
       for (int l = 0; l < nt; ++l) sv[b + l] = in.sv[u + l];
       std::memcpy(in.sv, sv, sizeof(sv));
     }
   }
-  z->has_bc = true;
+  // the inflow table is read when a queued launch runs: the work of every
+  // stream is finished before it changes (the copy alone would wait for the
+  // null stream only); the zone changes only when the copy has succeeded
+  HIP_TRY(hipDeviceSynchronize());
+  HIP_TRY(hipMemcpy(z->d_inflow, next.inflow, sizeof(next.inflow), hipMemcpyHostToDevice));
   z->bc_plan.swap(plan);
-  if (!z->bc_plan.empty())
-    HIP_TRY(hipMemcpy(z->d_bc_plan, z->bc_plan.data(), z->bc_plan.size() * sizeof(FaceBatch), hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(z->d_inflow, z->bc.inflow, sizeof(z->bc.inflow), hipMemcpyHostToDevice));
+  z->has_bc = true;
   return OSTC_OK;
 }
 
@@ -925,8 +923,8 @@ int ostc_limit_flow(ostc_ctx *c, ostc_zone *z, void *s) {
 int ostc_apply_bc(ostc_ctx *c, ostc_zone *z, void *s) {
   if (!c || !z) return fail(OSTC_ERR_ARG, "null argument");
   if (!z->has_bc) return OSTC_OK;
-  return ZONE_CALL(z, apply_bc(z->vf, c->dev, c->opts, z->bc_plan, z->d_bc_plan, z->d_inflow, S(s)),
-                   apply_bc(z->vd, c->dev, c->opts, z->bc_plan, z->d_bc_plan, z->d_inflow, S(s)));
+  return ZONE_CALL(z, apply_bc(z->vf, c->dev, c->opts, z->bc_plan, z->d_inflow, S(s)),
+                   apply_bc(z->vd, c->dev, c->opts, z->bc_plan, z->d_inflow, S(s)));
 }
 
 int ostc_inner_halo(ostc_ctx *c, ostc_zone **zones, int blk, const ostc_inner_face *f, void *s) {

@@ -273,19 +273,20 @@ __device__ __forceinline__ void one_face(const ZoneView<R> &z, const BatchFace &
   }
 }
 
-// One launch over the faces of a batch.  What a launch costs is latency: the
-// batch is read from device memory (kernel arguments live in host memory),
-// the workgroup's face by the grid's z (no divisions), and the face direction
-// is a template argument (no indexed registers): the code a wave walks
-// through once, uncached, is the time.
+// One launch over the faces of a batch.  The batch travels with the launch, as
+// the grid does, so that a launch that is queued or captured keeps the faces,
+// wall flags and wall temperatures it was made for.  What a launch costs is
+// latency: the workgroup's face follows from the grid's z (no divisions), and
+// the face direction is a template argument (no indexed registers): the code
+// a wave walks through once, uncached, is the time.
 template <typename R, int NS, int NT>
-__global__ __launch_bounds__(256) void k_faces(ZoneView<R> z, const FaceBatch *__restrict__ batch,
+__global__ __launch_bounds__(256) void k_faces(ZoneView<R> z, const FaceBatch batch,
                                                const ostc_param *__restrict__ p,
                                                const ostc_inflow *__restrict__ in) {
   int q = 0;
 #pragma unroll
-  for (int k = 1; k < kBatchFaces; ++k) q += (int)blockIdx.z >= batch->first[k];
-  const BatchFace &b = batch->face[q];
+  for (int k = 1; k < kBatchFaces; ++k) q += (int)blockIdx.z >= batch.first[k];
+  const BatchFace &b = batch.face[q];
   if ((int)blockIdx.x >= b.gx || (int)blockIdx.y >= b.gy) return;
   const uint3 blk = make_uint3(blockIdx.x, blockIdx.y, blockIdx.z - (unsigned)b.first);
   if (b.f.face == 0)
@@ -491,11 +492,10 @@ int plan_bc(const ostc_bc &bc, int ngg, std::vector<FaceBatch> &batches) {
 
 template <typename R>
 int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const std::vector<FaceBatch> &plan,
-             const FaceBatch *d_plan, const ostc_inflow *d_inflow, hipStream_t st) {
-  for (size_t q = 0; q < plan.size(); ++q) {
-    const dim3 grid((unsigned)plan[q].gx, (unsigned)plan[q].gy, (unsigned)plan[q].gz), block(64, 4, 1);
-    OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_faces<R, NS_, NT_>), grid, block, 0, st, z, d_plan + q, dp,
-                                             d_inflow));
+             const ostc_inflow *d_inflow, hipStream_t st) {
+  for (const FaceBatch &b : plan) {
+    const dim3 grid((unsigned)b.gx, (unsigned)b.gy, (unsigned)b.gz), block(64, 4, 1);
+    OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_faces<R, NS_, NT_>), grid, block, 0, st, z, b, dp, d_inflow));
     if (hipGetLastError() != hipSuccess) return OSTC_ERR_HIP;
   }
   return OSTC_OK;
@@ -547,9 +547,9 @@ int wall_friction_heatflux(const ZoneView<R> &z, double dyn_pressure, double *cf
 }
 
 template int apply_bc<float>(const ZoneView<float> &, const ostc_param *, const CellOpts &,
-                             const std::vector<FaceBatch> &, const FaceBatch *, const ostc_inflow *, hipStream_t);
+                             const std::vector<FaceBatch> &, const ostc_inflow *, hipStream_t);
 template int apply_bc<double>(const ZoneView<double> &, const ostc_param *, const CellOpts &,
-                              const std::vector<FaceBatch> &, const FaceBatch *, const ostc_inflow *, hipStream_t);
+                              const std::vector<FaceBatch> &, const ostc_inflow *, hipStream_t);
 template int inner_halo<float>(const ZoneView<float> &, const ZoneView<float> &, const ostc_param *,
                                const CellOpts &, const ostc_inner_face &, hipStream_t);
 template int inner_halo<double>(const ZoneView<double> &, const ZoneView<double> &, const ostc_param *,

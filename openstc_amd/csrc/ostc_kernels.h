@@ -133,7 +133,7 @@ struct FaceBatch {
 int plan_bc(const ostc_bc &bc, int ngg, std::vector<FaceBatch> &batches);
 template <typename R>
 int apply_bc(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, const std::vector<FaceBatch> &plan,
-             const FaceBatch *d_plan, const ostc_inflow *d_inflow, hipStream_t st);
+             const ostc_inflow *d_inflow, hipStream_t st);
 template <typename R>
 int inner_halo(const ZoneView<R> &z, const ZoneView<R> &t, const ostc_param *dp, const CellOpts &o,
                const ostc_inner_face &f, hipStream_t st);
