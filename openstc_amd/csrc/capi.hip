@@ -1338,7 +1338,8 @@ int ostc_surrogate_create(ostc_ctx *ctx, const ostc_surrogate_desc *desc, const 
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&S.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || S.cus <= 0)
-    S.cus = 256;
+    S.cus = ostc::kSurRows;
+  S.cus = std::min(S.cus, ostc::kSurRows);
   const size_t np = (size_t)S.n_params;
   hipError_t e = hipSuccess;
   auto A = [&](auto **p, size_t n) {
@@ -1355,6 +1356,7 @@ int ostc_surrogate_create(ostc_ctx *ctx, const ostc_surrogate_desc *desc, const 
   A(&S.bias, (size_t)ostc::kSurBias);
   A(&S.loss_w, 16);
   A(&S.stats, (size_t)S.cus * 4);
+  A(&S.listed, (size_t)ostc::kSurRows);
   if (max_batch > 0) {
     const size_t B = (size_t)max_batch;
     A(&S.a0, B * 16);

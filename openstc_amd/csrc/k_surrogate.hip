@@ -197,6 +197,7 @@ struct TrainOut {
 struct InferOut {
   double *dy;                    // [n][9]
   unsigned *rejected;            // [n]: each workgroup's rejected cells (less its first cell), from its first cell on
+  unsigned *listed;              // [kSurRows]: cells in each workgroup's list
   unsigned long long *stats;     // [stat_rows][4], a row per workgroup: its first cell, cells rejected for each reason
   int stat_rows;
   float *raw;                    // optional [n][16] standardised outputs
@@ -477,8 +478,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_sur_forward(SurParams s, Src src
     if (threadIdx.x < 4)
       io.stats[(long)blockIdx.x * 4 + threadIdx.x] =
           threadIdx.x == 0 ? (unsigned long long)wg0 : (unsigned long long)rejected[threadIdx.x];
-    if (blockIdx.x == 0)
+    if (threadIdx.x == 0) io.listed[blockIdx.x] = rejected[0];
+    if (blockIdx.x == 0) {
       for (int q = gridDim.x * 4 + threadIdx.x; q < io.stat_rows * 4; q += blockDim.x) io.stats[q] = 0;
+      for (int q = gridDim.x + threadIdx.x; q < kSurRows; q += blockDim.x) io.listed[q] = 0;
+    }
   }
 }
 
@@ -497,28 +501,50 @@ __device__ __forceinline__ int touch_tables(const ostc_param *__restrict__ p, in
 }
 
 // Plain point-implicit step on the cells that the checks rejected, 64 a wave:
-// the wave takes its share of one workgroup's list (written on the same XCD:
-// the grid is `per` times the forward's, a multiple of 8 where it is large).
-// What it costs is one step's latency as long as no SIMD has two waves of it,
-// so the lists are kept dense: rejected cells come in clusters, and with a
-// fixed run of cells for each wave some had to go round twice (1 M states, 1.8
-// % rejected: 48 us).
+// the waves take pieces of all workgroups' lists joined end to end, so that
+// neither a wave nor a round is partly filled.  Rejected cells come in clusters
+// (a list is a run of cells, in a zone a region of space): with waves bound to
+// a list, 2 % of a 256x192x128 zone in one region made a step of 2 617 us (1 251
+// with them spread out), since the waves of a few lists went round 48 times
+// while the others had none; now it is 1 225 us (1 234).  Every wave sums the lists' lengths
+// itself (four a lane and a wave scan).
 template <typename Src, bool RED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_sur_fallback(
     const ostc_param *__restrict__ p, Src src, const unsigned *__restrict__ rejected,
-    const unsigned long long *__restrict__ stats, int wgs, int per, double *__restrict__ dyo) {
+    const unsigned *__restrict__ listed, const unsigned long long *__restrict__ stats, int rows,
+    double *__restrict__ dyo) {
   __shared__ ConcGibbs tab_mem[RED ? kRedEntries * 64 : 1];
-  const int wg = (int)blockIdx.x % wgs, ln = threadIdx.x;
-  const unsigned long long *row = stats + (long)wg * 4;
-  const int m = (int)(row[1] + row[2] + row[3]), first = (int)blockIdx.x / wgs * 64;
-  if (first >= m) return;
+  __shared__ __attribute__((aligned(16))) unsigned upto[kSurRows];  // cells in the lists up to this one
+  __shared__ long first[kSurRows];     // first cell of each list's workgroup
+  static_assert(kSurRows == 4 * 64, "four lists a lane");
+  const int ln = threadIdx.x;
+  uint4 sum = reinterpret_cast<const uint4 *>(listed)[ln];
+  sum.y += sum.x;
+  sum.z += sum.y;
+  sum.w += sum.z;
+  unsigned at = sum.w;
+#pragma unroll
+  for (int d = 1; d < 64; d *= 2) {
+    const unsigned below = __shfl_up(at, d);
+    if (ln >= d) at += below;
+  }
+  const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)at, 63);
+  if (blockIdx.x * 64u >= total) return;
+  at -= sum.w;
+  reinterpret_cast<uint4 *>(upto)[ln] = make_uint4(at + sum.x, at + sum.y, at + sum.z, at + sum.w);
+#pragma unroll
+  for (int r = ln; r < kSurRows; r += 64) first[r] = r < rows ? (long)stats[(long)r * 4] : 0;
   if constexpr (RED) {
     const int warm = touch_tables(p, ln);
     asm volatile("" ::"v"(warm));
   }
-  const long wg0 = (long)row[0];
-  for (int q = first + ln; q < m; q += per * 64) {
-    const long c = wg0 + rejected[wg0 + q];
+  wave_sync();
+  for (unsigned q = blockIdx.x * 64u + ln; q < total; q += gridDim.x * 64u) {
+    int l = 0;  // the list of entry q: lists whose cells all come before it
+#pragma unroll
+    for (int d = kSurRows / 2; d > 0; d /= 2)
+      if (upto[l + d - 1] <= q) l += d;
+    const long wg0 = first[l], c = wg0 + rejected[wg0 + (q - (l ? upto[l - 1] : 0u))];
     double T, P, DT, Y[kNs];
     src.load(c, T, P, Y, DT);
     if constexpr (RED) {
@@ -733,7 +759,7 @@ int sur_pack(const SurState &st, hipStream_t s) {
 }
 
 template <typename Src, bool TRAIN, int CELLS, int TILES, int WAVES>
-static int launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
+static void launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
                            hipStream_t s) {
   const long wgs = (src.n + WAVES * CELLS - 1) / (WAVES * CELLS);
   const dim3 grid((unsigned)std::max<long>(1, std::min<long>(wgs, st.cus))), block(WAVES * 64);
@@ -744,26 +770,27 @@ static int launch_forward(const SurState &st, const Src &src, const TrainOut &tr
   else
     hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_GELU, CELLS, TILES, WAVES>), grid, block, 0, s,
                        st.params, src, wpk, st.bias, tr, io);
-  return (int)grid.x;
 }
 
 template <typename Src>
 static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, double *dy, float *raw,
                       hipStream_t s) {
   TrainOut tr{};
-  InferOut io{dy, st.rejected, st.stats, st.cus, raw};
+  InferOut io{dy, st.rejected, st.listed, st.stats, st.cus, raw};
   // batches that 64-cell passes would leave on part of the CUs: 16 cells a wave
-  const int wgs = src.n < 64L * kWaves * st.cus / 2 ? launch_forward<Src, false, 16, 1, 4>(st, src, tr, io, s)
-                                                    : launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
-  // one wave per 64 cells of a workgroup, at most two a SIMD
-  const int per = (int)std::min<long>(8, (src.n / wgs + 32 * kWaves + 63) / 64);
-  const dim3 fb_grid((unsigned)(wgs * per));
-  if (st.red)
-    hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.stats,
-                       wgs, per, dy);
+  if (src.n < 64L * kWaves * st.cus / 2)
+    launch_forward<Src, false, 16, 1, 4>(st, src, tr, io, s);
   else
-    hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.stats,
-                       wgs, per, dy);
+    launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
+  // one wave per 64 cells, as many as the registers let the device hold (two
+  // or one a SIMD); those past the number rejected end at once
+  const dim3 fb_grid((unsigned)std::min<long>((src.n + 63) / 64, (st.red ? 8L : 4L) * st.cus));
+  if (st.red)
+    hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.listed,
+                       st.stats, st.cus, dy);
+  else
+    hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.listed,
+                       st.stats, st.cus, dy);
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 

@@ -23,6 +23,10 @@ constexpr float kInvAtm = (float)(1.0 / 101325.0);
 constexpr float kBoxCox = 0.1f;
 constexpr float kInvBoxCox = 10.0f;
 constexpr float kAdamB1 = 0.9f, kAdamB2 = 0.999f, kAdamEps = 1e-8f;
+// Workgroups of the inference kernel at most (one per CU), each with a list of
+// rejected cells whose lengths a wave of the fallback kernel sums.
+constexpr int kSurRows = 256;
+
 // parameter layout: per layer W[out][in] row-major, then b[out]
 __host__ __device__ inline int sur_in_dim(int l) { return l == 0 ? kSurIn : kSurHidden; }
 __host__ __device__ inline int sur_out_dim(int l, int n_out) { return l == 4 ? n_out : kSurHidden; }
@@ -48,7 +52,7 @@ struct SurState {
   SurParams params{};
   int n_params = 0;
   bool red = false;  // the mechanism has reduced chemistry tables (fallback step)
-  int cus = 256;
+  int cus = kSurRows;  // at most kSurRows
   long max_batch = 0;
   long adam_step = 0;
   float *master = nullptr, *grad = nullptr, *m1 = nullptr, *m2 = nullptr, *wq = nullptr;
@@ -57,6 +61,7 @@ struct SurState {
   float *loss_w = nullptr; // 16
   unsigned *rejected = nullptr;  // [fb_cap] cells the checks rejected, by forward workgroup
   long fb_cap = 0;               // cells `rejected` is sized for
+  unsigned *listed = nullptr;    // [kSurRows] cells in each list
   unsigned long long *stats = nullptr;  // [cus][4], a row per workgroup: its first cell, cells rejected by reason
   // training buffers (max_batch rows)
   float *a0 = nullptr, *z = nullptr, *a = nullptr, *yout = nullptr, *g5 = nullptr;
