@@ -1334,7 +1334,6 @@ int ostc_surrogate_create(ostc_ctx *ctx, const ostc_surrogate_desc *desc, const 
   S.params = sur_params(*desc);
   S.n_params = ostc::sur_n_params(desc->n_out);
   S.max_batch = max_batch;
-  S.red = ctx->opts.red;
   int dev = 0;
   (void)hipGetDevice(&dev);
   if (hipDeviceGetAttribute(&S.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || S.cus <= 0)
@@ -1422,7 +1421,7 @@ int ostc_surrogate_step(ostc_surrogate *s, long n, const double *t, const double
   if (!s || n < 0 || (n > 0 && (!t || !p || !y || !dt || !dy))) return fail(OSTC_ERR_ARG, "bad arguments");
   int st = sur_ensure_fallback(s, n);
   if (st) return st;
-  st = ostc::sur_infer_batch(s->st, s->ctx->dev, n, t, p, y, dt, dy, nullptr, S(strm));
+  st = ostc::sur_infer_batch(s->st, s->ctx->dev, s->ctx->opts.red, n, t, p, y, dt, dy, nullptr, S(strm));
   if (st) return fail(st, "surrogate inference launch failed");
   return sur_read_stats(s, n, stats, S(strm));
 }
@@ -1432,7 +1431,7 @@ int ostc_surrogate_forward(ostc_surrogate *s, long n, const double *t, const dou
   if (!s || n < 0 || (n > 0 && (!t || !p || !y || !dt || !raw || !dy))) return fail(OSTC_ERR_ARG, "bad arguments");
   int st = sur_ensure_fallback(s, n);
   if (st) return st;
-  st = ostc::sur_infer_batch(s->st, s->ctx->dev, n, t, p, y, dt, dy, raw, S(strm));
+  st = ostc::sur_infer_batch(s->st, s->ctx->dev, s->ctx->opts.red, n, t, p, y, dt, dy, raw, S(strm));
   return st ? fail(st, "surrogate inference launch failed") : OSTC_OK;
 }
 
@@ -1474,8 +1473,8 @@ int ostc_chem_zone_step(ostc_ctx *c, ostc_zone *z, ostc_surrogate *s, int mode, 
   }
   st = sur_ensure_fallback(s, n);
   if (st) return st;
-  st = fp64(z) ? ostc::sur_infer_zone(s->st, c->dev, z->vd, dy, S(strm))
-               : ostc::sur_infer_zone(s->st, c->dev, z->vf, dy, S(strm));
+  st = fp64(z) ? ostc::sur_infer_zone(s->st, c->dev, c->opts.red, z->vd, dy, S(strm))
+               : ostc::sur_infer_zone(s->st, c->dev, c->opts.red, z->vf, dy, S(strm));
   if (st) return fail(st, "surrogate inference launch failed");
   return sur_read_stats(s, n, stats, S(strm));
 }

@@ -773,7 +773,7 @@ static void launch_forward(const SurState &st, const Src &src, const TrainOut &t
 }
 
 template <typename Src>
-static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, double *dy, float *raw,
+static int infer_impl(const SurState &st, const ostc_param *dp, bool red, const Src &src, double *dy, float *raw,
                       hipStream_t s) {
   TrainOut tr{};
   InferOut io{dy, st.rejected, st.listed, st.stats, st.cus, raw};
@@ -784,8 +784,8 @@ static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, 
     launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
   // one wave per 64 cells, as many as the registers let the device hold (two
   // or one a SIMD); those past the number rejected end at once
-  const dim3 fb_grid((unsigned)std::min<long>((src.n + 63) / 64, (st.red ? 8L : 4L) * st.cus));
-  if (st.red)
+  const dim3 fb_grid((unsigned)std::min<long>((src.n + 63) / 64, (red ? 8L : 4L) * st.cus));
+  if (red)
     hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.listed,
                        st.stats, st.cus, dy);
   else
@@ -794,17 +794,17 @@ static int infer_impl(const SurState &st, const ostc_param *dp, const Src &src, 
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
-int sur_infer_batch(const SurState &st, const ostc_param *dp, long n, const double *t, const double *p,
+int sur_infer_batch(const SurState &st, const ostc_param *dp, bool red, long n, const double *t, const double *p,
                     const double *y, const double *dt, double *dy, float *raw, hipStream_t s) {
   if (n <= 0) return OSTC_OK;
   BatchSrc src{t, p, y, dt, nullptr, n};
-  return infer_impl(st, dp, src, dy, raw, s);
+  return infer_impl(st, dp, red, src, dy, raw, s);
 }
 
 template <typename R>
-int sur_infer_zone(const SurState &st, const ostc_param *dp, const ZoneView<R> &z, double *dy, hipStream_t s) {
+int sur_infer_zone(const SurState &st, const ostc_param *dp, bool red, const ZoneView<R> &z, double *dy, hipStream_t s) {
   ZoneSrc<R> src{z.bv, z.sv, z.dt, z.mx, z.my, z.g, z.nx, z.ny, z.plane, (long)z.mx * z.my * z.mz};
-  return infer_impl(st, dp, src, dy, nullptr, s);
+  return infer_impl(st, dp, red, src, dy, nullptr, s);
 }
 
 template <typename R>
@@ -818,9 +818,9 @@ int zone_plain_chem(const ostc_param *dp, bool red, const ZoneView<R> &z, double
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 
-template int sur_infer_zone<float>(const SurState &, const ostc_param *, const ZoneView<float> &, double *,
+template int sur_infer_zone<float>(const SurState &, const ostc_param *, bool, const ZoneView<float> &, double *,
                                    hipStream_t);
-template int sur_infer_zone<double>(const SurState &, const ostc_param *, const ZoneView<double> &, double *,
+template int sur_infer_zone<double>(const SurState &, const ostc_param *, bool, const ZoneView<double> &, double *,
                                     hipStream_t);
 template int zone_plain_chem<float>(const ostc_param *, bool, const ZoneView<float> &, double *, hipStream_t);
 template int zone_plain_chem<double>(const ostc_param *, bool, const ZoneView<double> &, double *, hipStream_t);

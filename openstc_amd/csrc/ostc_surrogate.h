@@ -51,7 +51,6 @@ struct SurParams {
 struct SurState {
   SurParams params{};
   int n_params = 0;
-  bool red = false;  // the mechanism has reduced chemistry tables (fallback step)
   int cus = kSurRows;  // at most kSurRows
   long max_batch = 0;
   long adam_step = 0;
@@ -121,10 +120,11 @@ __device__ __forceinline__ int sur_check_change(const SurParams &s, const float 
 }
 
 int sur_pack(const SurState &st, hipStream_t s);
-int sur_infer_batch(const SurState &st, const ostc_param *dp, long n, const double *t, const double *p,
+// red: dp's mechanism has reduced chemistry tables (ChemRed; the fallback step)
+int sur_infer_batch(const SurState &st, const ostc_param *dp, bool red, long n, const double *t, const double *p,
                     const double *y, const double *dt, double *dy, float *raw, hipStream_t s);
 template <typename R>
-int sur_infer_zone(const SurState &st, const ostc_param *dp, const ZoneView<R> &z, double *dy, hipStream_t s);
+int sur_infer_zone(const SurState &st, const ostc_param *dp, bool red, const ZoneView<R> &z, double *dy, hipStream_t s);
 template <typename R>
 int zone_plain_chem(const ostc_param *dp, bool red, const ZoneView<R> &z, double *dy, hipStream_t s);
 int sur_gradients(const SurState &st, long nb, const double *t, const double *p, const double *y, const double *dt,

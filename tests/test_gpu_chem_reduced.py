@@ -16,7 +16,8 @@ import oracle_ffi as O
 from harness import Pair, interior, scaled_err
 from openstc_amd import _lib as L
 from openstc_amd import cases
-from openstc_amd.runtime import Context
+from openstc_amd.runtime import Context, Simulation
+from openstc_amd.surrogate import DeviceArray, Surrogate
 from test_gpu_chem import Dev, states
 
 pytestmark = pytest.mark.gpu
@@ -112,3 +113,32 @@ def test_time_step(name, precision, tol):
         print(f"[gpu-red] {f} err {e:.2e}", flush=True)
         assert e < tol, (f, e)
     pr.gpu.close()
+
+
+@pytest.mark.parametrize("own,zone", [("as shipped", "inert catalyst"), ("inert catalyst", "as shipped")])
+@pytest.mark.parametrize("precision", [L.FP64, L.FP32])
+def test_fallback_takes_the_zones_mechanism(own, zone, precision):
+    """A surrogate may step a zone of another context: the cells it rejects
+    take the plain step of the zone's mechanism, with or without the tables."""
+    print(f"[gpu-red] surrogate of '{own}' on a zone of '{zone}', precision {precision}", flush=True)
+    sur = Surrogate.load(Context(with_flow(mechanism(own))), t_max=1.0)  # rejects every state
+    case = cases.mixing_layer(mx=21, my=18, mz=9, precision=precision)
+    mech = mechanism(zone)
+    for k in ARRAYS + ("stoi_f", "stoi_b", "third_body_coeff"):
+        getattr(case.param, k)[:] = list(getattr(mech, k))
+    case.param.n_reac = mech.n_reac
+    sim = Simulation(case)
+    sim.initialize_computation()
+    sim.step()
+    n = 21 * 18 * 9
+    dy, st = [DeviceArray(nbytes=n * 9 * 8) for _ in range(2)], (C.c_longlong * 4)()
+    for mode in (0, 1):
+        L.check(sim.ctx.lib.ostc_chem_zone_step(sim.ctx.h, sim.zones[0].h, sur.h if mode else None, mode, dy[mode].p,
+                                                st if mode else None, None), "zone chemistry")
+    plain, got = (d.get(np.float64, (n, 9)) for d in dy)
+    assert list(st) == [n, n, 0, 0]
+    assert np.abs(plain).max() > 0 and np.array_equal(got, plain)
+    for d in dy:
+        d.free()
+    sur.close()
+    sim.close()
