@@ -1249,14 +1249,16 @@ int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpt
     } else {
       OSTC_DISPATCH_NSNT(o, hipLaunchKernelGGL((k_dq0<R, NS_, NT_, false>), g.grid, g.block, 0, st, z, dp));
     }
+    int r = last_err();
+    if (r == OSTC_OK && o.ns > 0 && o.dplur_steps > 0) r = dplur_scalars(z, dp, o, st);
     prof_mark(P_DQ0, st, false);
-    if (last_err()) return OSTC_ERR_HIP;
+    if (r) return r;
   }
   if (o.dplur_steps == 0) {
     *result = z.dq0;
     return OSTC_OK;
   }
-  return dplur_sweeps(z, dp, o, st, chem_late, false, result);
+  return dplur_sweeps(z, dp, o, st, chem_late, result);
 }
 
 // check_slot >= 0: also classify every cell for limit_flow into repair-list

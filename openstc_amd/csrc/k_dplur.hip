@@ -64,7 +64,7 @@ __device__ __forceinline__ R pressure_increment(const ostc_param *__restrict__ p
 
 // h and s of the stored increment d (mixtures whose d was written by a kernel
 // that does not form them)
-template <typename R, int NS, int NT, bool H>
+template <typename R, int NS, bool H>
 __global__ __launch_bounds__(256) void k_dplur_scalars(ZoneView<R> z, const ostc_param *__restrict__ p,
                                                        const R *__restrict__ din, R *__restrict__ s_out) {
   const uint3 b = xcd_block();
@@ -568,16 +568,6 @@ inline int dplur_chunk_planes(int tiles, int mz, int resident) {
 
 inline int last_err() { return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP; }
 
-template <typename R, int NS, int NT>
-int scalars(const ZoneView<R> &z, const ostc_param *dp, const R *d, R *s, bool h, hipStream_t st) {
-  const auto g = cell_grid(z.mx, z.my, z.mz);
-  if (h)
-    hipLaunchKernelGGL((k_dplur_scalars<R, NS, NT, true>), g.grid, g.block, 0, st, z, dp, d, s);
-  else
-    hipLaunchKernelGGL((k_dplur_scalars<R, NS, NT, false>), g.grid, g.block, 0, st, z, dp, d, s);
-  return last_err();
-}
-
 // the EPI block solve of a mechanism without reduced tables
 template <typename R, int NS>
 int chem_solve(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, bool tiled, R *out, hipStream_t st) {
@@ -621,7 +611,7 @@ int sweeps_air(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hi
 // mixtures: dq0 stays, dqk and dq take the increments in turn
 template <typename R, int NS, int NT>
 int sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool chem_late,
-           bool scalars_ready, R **result) {
+           R **result) {
   const bool chem = o.mix_model == OSTC_FR, epi = chem && o.chem == 1;
   const bool reduced = epi && chem_late && o.red;
   const auto g = cell_grid(z.mx, z.my, z.mz);
@@ -629,8 +619,6 @@ int sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStr
   const unsigned jb = std::max(1u, 24u / g.grid.x);
   R *in = z.dq0, *out = z.dqk;
   R *s_in = z.imp + z.plane, *s_out = s_in + z.plane;
-  if (!scalars_ready)
-    if (int r = scalars<R, NS, NT>(z, dp, in, s_in, true, st)) return r;
   for (int q = 0; q < o.dplur_steps; ++q) {
     const bool last = q + 1 == o.dplur_steps;
     R *so = last ? nullptr : s_out;
@@ -657,7 +645,10 @@ int sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStr
     if (epi && !reduced) {
       prof_mark(P_DPLUR_CHEM, st, true);
       int r = chem_solve<R, NS>(z, dp, o, chem_late, out, st);
-      if (r == OSTC_OK && !last) r = scalars<R, NS, NT>(z, dp, out, s_out, false, st);
+      if (r == OSTC_OK && !last) {
+        hipLaunchKernelGGL((k_dplur_scalars<R, NS, false>), g.grid, g.block, 0, st, z, dp, (const R *)out, s_out);
+        r = last_err();
+      }
       prof_mark(P_DPLUR_CHEM, st, false);
       if (r) return r;
     }
@@ -672,19 +663,34 @@ int sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStr
 }  // namespace
 
 template <typename R>
+int dplur_scalars(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st) {
+  const auto g = cell_grid(z.mx, z.my, z.mz);
+  R *s = z.imp + z.plane;
+  if (o.ns == 9)
+    hipLaunchKernelGGL((k_dplur_scalars<R, 9, true>), g.grid, g.block, 0, st, z, dp, (const R *)z.dq0, s);
+  else if (o.ns == 20)
+    hipLaunchKernelGGL((k_dplur_scalars<R, 20, true>), g.grid, g.block, 0, st, z, dp, (const R *)z.dq0, s);
+  else
+    return OSTC_ERR_ARG;
+  return last_err();
+}
+
+template <typename R>
 int dplur_sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool chem_late,
-                 bool scalars_ready, R **result) {
+                 R **result) {
   if (o.ns == 0) return o.nt == 2 ? sweeps_air<R, 2>(z, dp, o, st, result) : sweeps_air<R, 0>(z, dp, o, st, result);
-  if (o.ns == 9 && o.nt == 2) return sweeps<R, 9, 2>(z, dp, o, st, chem_late, scalars_ready, result);
-  if (o.ns == 9 && o.nt == 0) return sweeps<R, 9, 0>(z, dp, o, st, chem_late, scalars_ready, result);
-  if (o.ns == 20 && o.nt == 2) return sweeps<R, 20, 2>(z, dp, o, st, chem_late, scalars_ready, result);
-  if (o.ns == 20 && o.nt == 0) return sweeps<R, 20, 0>(z, dp, o, st, chem_late, scalars_ready, result);
+  if (o.ns == 9 && o.nt == 2) return sweeps<R, 9, 2>(z, dp, o, st, chem_late, result);
+  if (o.ns == 9 && o.nt == 0) return sweeps<R, 9, 0>(z, dp, o, st, chem_late, result);
+  if (o.ns == 20 && o.nt == 2) return sweeps<R, 20, 2>(z, dp, o, st, chem_late, result);
+  if (o.ns == 20 && o.nt == 0) return sweeps<R, 20, 0>(z, dp, o, st, chem_late, result);
   return OSTC_ERR_ARG;
 }
 
+template int dplur_scalars<float>(const ZoneView<float> &, const ostc_param *, const CellOpts &, hipStream_t);
+template int dplur_scalars<double>(const ZoneView<double> &, const ostc_param *, const CellOpts &, hipStream_t);
 template int dplur_sweeps<float>(const ZoneView<float> &, const ostc_param *, const CellOpts &, hipStream_t, bool,
-                                 bool, float **);
+                                 float **);
 template int dplur_sweeps<double>(const ZoneView<double> &, const ostc_param *, const CellOpts &, hipStream_t, bool,
-                                  bool, double **);
+                                  double **);
 
 }  // namespace ostc

@@ -80,11 +80,13 @@ int local_time_step(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &
 template <typename R>
 int implicit_treatment(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, R **result,
                        bool chem_late = false);
-// k_dplur.hip: the sweeps of implicit_treatment from dq0 (mixtures) or dq
-// (air); scalars_ready: h and s of dq0 are in z.imp
+// k_dplur.hip: the sweeps of implicit_treatment from dq (air) or from dq0 and
+// its h and s in z.imp (mixtures), which dplur_scalars forms
+template <typename R>
+int dplur_scalars(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st);
 template <typename R>
 int dplur_sweeps(const ZoneView<R> &z, const ostc_param *dp, const CellOpts &o, hipStream_t st, bool chem_late,
-                 bool scalars_ready, R **result);
+                 R **result);
 // check_slot >= 0: also classify every cell for limit_flow into repair-list
 // slot (check_slot & 1); then call limit_flow with the same slot.  Time steps
 // alternate the slot.
