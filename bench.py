@@ -139,11 +139,14 @@ def alg_bytes_per_cell(p, esize: int) -> dict:
     na = sum(1 for l in range(ns) if any(p.stoi_f[r * L.MAX_SPEC + l] or p.stoi_b[r * L.MAX_SPEC + l]
                                           for r in range(p.n_reac)))
     npw = (na + 7) // 8
-    # EPI under DPLUR on the 9-species kernels (at most 20 reactions): the
-    # source kernel forms the SST source and the local time step only, and
-    # the chemistry follows the fluxes in the dq0 stage, which also stores
-    # the chemistry block's LU factors
-    fac = epi and ns == 9 and p.n_reac <= 20 and p.implicit_method == 1 and na > 0
+    # EPI under DPLUR on the 9-species kernels (mechanisms with reduced
+    # chemistry tables, others of at most 20 reactions): the source kernel
+    # forms the SST source and the local time step only, and the chemistry
+    # follows the fluxes in the dq0 stage, which also stores the chemistry
+    # block's factors: 6x6 and 6x2 with the tables, na x na without
+    red = epi and reduced_tables(p)
+    fac = epi and ns == 9 and (red or p.n_reac <= 20) and p.implicit_method == 1 and na > 0
+    nfac = 48 if red and fac else na * na
     out = {}
 
     def put(stage, n_bulk, n_f64=0, n_i32=0):
@@ -192,29 +195,43 @@ def alg_bytes_per_cell(p, esize: int) -> dict:
         put("source", src, njac)
     # local time step: metric 9, u,v,w, rho, c [mu] [mu_t] [gamma] -> spectral radii 3, dt
     put("local_dt", 9 + 3 + 2 + (1 if visc else 0) + (1 if rans else 0) + (1 if ns else 0) + 4)
-    # DQ0 (reacting zones; non-reacting zones form dq0 in the first sweep):
-    # dq, dt, spectral radii 3, [J_t 2] -> dq0; the reacting species' block of
-    # the Jacobian read, its LU factors + packed pivots written (fac: the
-    # factors and pivots read)
+    # DQ0 (mixtures; air zones form dq0 in the first sweep): dq, dt, spectral
+    # radii 3, [J_t 2] -> dq0; the reacting species' block of the Jacobian
+    # read, its LU factors + packed pivots written.  The stage ends with the
+    # scalars of dq0 that the sweeps gather: its flow and species rows, Y, u,
+    # v, w, |V|, T, gamma -> total enthalpy, pressure increment
+    dq0 = nv + 1 + 3 + (2 if rans else 0) + nv
+    sca = 5 + ns + 6
+    ready = sca + ns + 2 if ns and p.dplur_inner_step > 0 else 0
     if fac:
-        # the chemistry after the fluxes with dq0: rho, T, Y, J, dq, dt,
-        # spectral radii 3, [J_t 2] -> dq0, the reduced block's factors (6x6
-        # and 6x2) + packed pivots
-        put("dplur_dq0", 2 + ns + 1 + nv + 1 + 3 + (2 if rans else 0) + nv, 48, npw)
+        # the chemistry after the fluxes with dq0: also rho, T, Y, J
+        put("dplur_dq0", dq0 + 2 + ns + 1 + ready, nfac, npw)
     elif epi:
-        put("dplur_dq0", nv + 1 + 3 + (2 if rans else 0) + nv, 2 * na * na, npw)
+        put("dplur_dq0", dq0 + ready, 2 * na * na, npw)
     else:
-        put("dplur_dq0", nv + 1 + 3 + (2 if rans else 0) + nv, njac)
+        put("dplur_dq0", dq0 + ready, njac)
     # one sweep, air: din, sv, u,v,w,|V|, p, rho, metric 9, spectral radii 3,
-    # dt, dq0, [J_t 2] -> dout; a mixture reads the total enthalpy and the
-    # pressure increment in place of |V|, T and gamma and writes the next
-    # sweep's pressure increment (T and gamma read for it), and with EPI it
-    # reads the block's factors and pivots
-    sweep = nv + nsc + 4 + 2 + 9 + 3 + 1 + nv + (2 if rans else 0) + nv
-    if epi:
-        put("dplur_sweep", sweep + 2, 48 if fac else na * na, npw)
+    # dt, dq0, [J_t 2] -> dout.  A mixture gathers the total enthalpy and the
+    # pressure increment instead of p and rho, and all sweeps but the last
+    # read |V|, T and gamma and write the next one's pressure increment.  EPI:
+    # with reduced tables the block is solved in the sweep (its factors and
+    # pivots read); without them the sweep leaves the species rows' sums (no
+    # species rows of dq0 read), and dplur_chem solves them in place (sums,
+    # dq0's species rows, dt, factors, pivots, the spectral radii 3 where a
+    # species does not react) and forms the pressure increment
+    more = (p.dplur_inner_step - 1) / max(1, p.dplur_inner_step)
+    sweep = nv + nsc + 3 + 2 + 9 + 3 + 1 + nv + (2 if rans else 0) + nv
+    if ns == 0:
+        sweep += 1
+    elif not epi or (red and fac):
+        sweep += 4 * more
+    if not epi:
+        put("dplur_sweep", sweep, ns if chem else 0)
+    elif red and fac:
+        put("dplur_sweep", sweep, nfac, npw)
     else:
-        put("dplur_sweep", sweep + (2 if ns else 0), ns if chem else 0)
+        put("dplur_sweep", sweep - ns)
+        put("dplur_chem", 3 * ns + 1 + (3 if na < ns else 0) + (sca + 1) * more, na * na, npw)
     put("dplur_sweep_first", sweep)   # reads dq in place of dq0 and writes dq0 in place of reading it
     # update: cv, dq, dt, J [T: the Newton start] -> cv, bv 6, sv, |V|
     put("update", nv + nv + 2 + (1 if ns else 0) + nv + 6 + nsc + 1)
@@ -222,6 +239,25 @@ def alg_bytes_per_cell(p, esize: int) -> dict:
     # gamma, c, mu, lambda, rho*D_k, Mach
     put("properties", 6 if ns == 0 else 1 + ns + 1 + 5 + ns + 1)
     return out
+
+
+def reduced_tables(p) -> bool:
+    """Whether the library keeps the EPI block of this mechanism reduced by its
+    conserved elements: nine species, at most three molecules on a side of a
+    reaction, at most six independent rows of net coefficients among the
+    reacting species and at most two dependent ones."""
+    import numpy as np
+
+    from openstc_amd import _lib as L
+
+    ns, nr = p.n_spec, p.n_reac
+    if ns != 9 or nr < 1:
+        return False
+    f, b = (np.array(a[:]).reshape(-1, L.MAX_SPEC)[:nr, :ns] for a in (p.stoi_f, p.stoi_b))
+    if min(f.min(), b.min()) < 0 or max(f.sum(1).max(), b.sum(1).max()) > 3:
+        return False
+    kept = int(np.linalg.matrix_rank(b - f))
+    return 1 <= kept <= 6 and int(((f != 0) | (b != 0)).any(0).sum()) - kept <= 2
 
 
 def plain_chem_flop_per_cell(p) -> int:
@@ -340,7 +376,7 @@ def time_leg(case, steps: int, warmup: int, stage_steps: int):
                 # per iteration = zones x repetitions (DPLUR sweeps)
                 per_it = cnt_s[i] / stage_steps
                 reps = 1
-                if n == "dplur_sweep":
+                if n in ("dplur_sweep", "dplur_chem"):
                     reps = p.dplur_inner_step - (1 if any(x == "dplur_sweep_first" and cnt_s[j] for j, x in
                                                           enumerate(names)) and n == "dplur_sweep" else 0)
                 byts = alg[n] * cells * reps / per_it
