@@ -45,27 +45,33 @@ METRIC = "Mcell-iter/s (flux+SST+chem+DPLUR), %HBM peak; surrogate vs plain chem
 # FETCH_SIZE and WRITE_SIZE on these workloads (FETCH_SIZE scaled x2.0 and
 # WRITE_SIZE x1.0, the factors a 512 MiB copy kernel gives).  Keyed by
 # (workload, stage); the summary with the commands is
-# profiles/kernels_fourblock_jet_4x256x192x128_plate_mixing_layer.md.
-# Re-measured whenever the kernel changes; a stage without an entry reports
-# null.
+# profiles/kernels_counters_gather_sweeps_jet_mixing_plate.md.  Re-measured
+# whenever the kernel changes; a stage without an entry reports null.  The
+# dq0 stage of a mixture is two kernels.
 MEASURED_TRAFFIC = {
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "source"): 1061.4e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_i"): 3578.1e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_j"): 4034.7e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_k"): 3071.3e6,
-    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "update"): 1767.5e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "dplur_sweep"): 7192.3e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "dplur_dq0"): 4597.1e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "source"): 1056.9e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_i"): 3576.3e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_j"): 4011.9e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "flux_k"): 3045.2e6,
+    ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "update"): 1767.3e6,
     ("h2_jet_vitiated_crossflow_fr_sst_4x256x192x128", "properties"): 730.5e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "dplur_sweep"): 1836.8e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "dplur_dq0"): 1253.8e6,
     ("h2air_mixing_layer_fr_epi_dplur", "source"): 144.8e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "flux_i"): 671.2e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "flux_j"): 838.4e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "flux_k"): 743.6e6,
-    ("h2air_mixing_layer_fr_epi_dplur", "update"): 442.8e6,
-    ("sst_flat_plate_dplur", "dplur_sweep"): 480.9e6,
-    ("sst_flat_plate_dplur", "dplur_sweep_first"): 499.3e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "flux_i"): 670.9e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "flux_j"): 839.8e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "flux_k"): 743.3e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "update"): 443.9e6,
+    ("h2air_mixing_layer_fr_epi_dplur", "properties"): 209.9e6,
+    ("sst_flat_plate_dplur", "dplur_sweep"): 484.5e6,
+    ("sst_flat_plate_dplur", "dplur_sweep_first"): 509.7e6,
     ("sst_flat_plate_dplur", "flux_ij"): 358.6e6,
-    ("sst_flat_plate_dplur", "flux_k"): 402.3e6,
-    ("sst_flat_plate_dplur", "source"): 300.8e6,
-    ("sst_flat_plate_dplur", "update"): 273.5e6,
+    ("sst_flat_plate_dplur", "flux_k"): 402.5e6,
+    ("sst_flat_plate_dplur", "source"): 305.4e6,
+    ("sst_flat_plate_dplur", "update"): 275.3e6,
+    ("sst_flat_plate_dplur", "properties"): 56.9e6,
 }
 
 

@@ -4,9 +4,12 @@
 //
 // Every cell takes from each of its six neighbours inside the block
 //   +-1/2 (A_dir(q) d(q) +- rho_dir(q) d(q)),
-// with the convective Jacobian A applied to the neighbour's increment d.  One
-// thread owns one cell and gathers the six terms from memory: no shared
-// memory, no barrier, 4-8 waves per SIMD to hide the loads behind.  A term is
+// with the convective Jacobian A applied to the neighbour's increment d.  In a
+// mixture one thread owns one cell and gathers the six terms from memory, with
+// no barrier and 3-8 waves per SIMD to hide the loads behind (53-132 vector
+// registers on the 9-species kernels; the variant that solves the reduced
+// species block re-orders its rows through 9 KB of LDS a workgroup, 18 KB in
+// FP64).  Air marches tiles through k instead (below).  A term is
 // two multiply-adds a row once three numbers of the neighbour are known: the
 // contravariant velocity, b1 = k.d(rho V) - U d(rho), and the pressure
 // increment s(q) (b2 + b3 - b4 of the reference), which for a mixture needs

@@ -15,13 +15,13 @@
 // inside each 32-wide k chunk is permuted consistently in the packed weights,
 // so activations never leave registers between layers.
 //
-// The forward kernel writes the standardised outputs straight from the MFMA
-// accumulators; a second, high-occupancy kernel (one thread per cell) decodes
-// them, runs the checks and stores dY.  In the fused form the decode's global
-// loads, stores and list atomics stalled the low-occupancy MLP waves for as
-// long as the MLP itself.  Cells that fail the input-range, output-range or
-// element-balance checks are appended to a list and re-done by the FP64 plain
-// integrator in a third kernel (no serialisation inside a wavefront).
+// Two launches a step.  The forward kernel also decodes the outputs, runs the
+// checks and stores dY, one lane per cell of a pass, from what the pass still
+// holds in registers and LDS; the decoding reads nothing from memory and the
+// cells that fail the input-range, output-range or element-balance checks take
+// one LDS atomic a pass, so it does not hold the MLP's few waves up.  They form
+// a list per workgroup, and the second kernel re-does the lists, joined end to
+// end, with the FP64 plain integrator, 64 cells a wave.
 //
 // Training: the same forward kernel (saving pre-activations and BF16-rounded
 // activations), a weighted-MSE gradient kernel, FP32-MFMA
@@ -506,8 +506,8 @@ __device__ __forceinline__ int touch_tables(const ostc_param *__restrict__ p, in
 // (a list is a run of cells, in a zone a region of space): with waves bound to
 // a list, 2 % of a 256x192x128 zone in one region made a step of 2 617 us (1 251
 // with them spread out), since the waves of a few lists went round 48 times
-// while the others had none; now it is 1 225 us (1 234).  Every wave sums the lists' lengths
-// itself (four a lane and a wave scan).
+// while the others had none; now it is 1 225 us (1 234).  Every wave sums the
+// lists' lengths itself (four a lane and a wave scan).
 template <typename Src, bool RED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_sur_fallback(
     const ostc_param *__restrict__ p, Src src, const unsigned *__restrict__ rejected,

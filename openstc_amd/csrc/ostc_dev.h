@@ -100,7 +100,8 @@ __device__ __forceinline__ T dmax(T a, T b) { return a > b ? a : b; }
 
 // An element at a 32-bit byte offset from a wave-uniform base: the load keeps
 // its base in scalar registers and one address register serves every plane.
-// A plane of 2^32 bytes cannot be reached: a zone has at least 60 of them.
+// For the mixture sweeps: their zones have more than 100 planes, so one of
+// 2^32 bytes would take more memory than the device has.
 template <typename R>
 __device__ __forceinline__ R at(const R *base, unsigned off) {
   return *reinterpret_cast<const R *>(reinterpret_cast<const char *>(base) + off);

@@ -86,6 +86,13 @@ constexpr size_t kChemF64Offset = (kThermoF32Offset + sizeof(ThermoF32) + 255) /
 // mechanism with fewer of either fills the remaining slots with species that
 // do not react (zero rows and columns of J, a zero row of L); it has enough of
 // those, since 9 - n_act >= (6 - kept) + (2 - dependent) + 1 for n_act <= 8.
+// Rounding of the point step against 80-bit sums, 10 000 random compositions
+// at 300-3500 K, 0.1-20 atm, time steps 1e-9 to 1e-3 s, relative to a state's
+// largest change: median 6e-15, 99 % within 3e-11 (whole block 1.2e-14 and
+// 1e-10).  A dependent species carries the error of the largest change
+// whatever its own: O2 left over in burnt gas (10 000 states, mass fractions
+// down to 1e-14, time steps below 1e-7 s) is off by 2e-14 of its own change in
+// the median and by 3e-7 in one state of a hundred (whole block 2e-15, 2e-14).
 constexpr int kRedKept = 6, kRedDep = 2, kRedSlots = kRedKept + kRedDep, kRedSpec = 9;
 constexpr int kRedFactors = kRedKept * kRedSlots;  // stored per cell: A's factors, then C
 constexpr int kRedOne = kRedSpec;                  // table entry with c = 1, g = 0
