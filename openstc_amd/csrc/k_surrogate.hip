@@ -243,9 +243,9 @@ __device__ __forceinline__ int tile_out(int kc) { return 104 + kc; }
 // rate): 84 % of the issue slots at 1 M cells.  The layers run on 32 cells at
 // a time so that the matrix results of one 32-unit chunk can be activated
 // while the next chunk's products run.  With a decode kernel behind it and the
-// outputs in memory between them the step took 443 us at 1.5 M cells, now
-// 340.  TRAIN and small batches take 16 cells per wave: 4 096 samples are then
-// 64 workgroups instead of 6 (loss gradients 309 -> 222 us).
+// outputs in memory between them the step took 444 us at 1.5 M cells, now
+// 347.  TRAIN and small batches take 16 cells per wave: 4 096 samples are then
+// 64 workgroups instead of 6 (loss gradients 309 -> 219 us).
 template <typename Src, bool TRAIN, int ACT, int CELLS, int TILES, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void k_sur_forward(SurParams s, Src src, const bf16x8 *__restrict__ wpk,
                                                             const float *__restrict__ bias, TrainOut tr,

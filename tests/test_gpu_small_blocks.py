@@ -55,3 +55,35 @@ def test_faces(shape):
     print(f"[gpu-small] err {e:.2e}", flush=True)
     assert e < 1e-9
     pr.close()
+
+
+@pytest.mark.parametrize("patches", [2, 5])
+@pytest.mark.parametrize("mz", [5, 11])
+def test_faces_in_patches(patches, mz):
+    """Each face of a plate cut into patches, 10 and 30 faces a program: runs of
+    disjoint ones longer than a launch takes, and between them faces that meet
+    at an edge and keep their order (5 planes: the k faces meet as well)."""
+    print(f"[gpu-small] plate 24x20x{mz}, {patches} patches a face", flush=True)
+    case = cases.sst_plate(24, 20, mz, precision=L.FP64, cfl=2.0, perturb=True)
+    whole, bc = case.blocks[0].bc, L.BC()
+    bc.inflow, bc.wall = whole.inflow, whole.wall
+    for f in range(whole.n_face):
+        src = whole.face[f]
+        along = 1 if src.face == 0 else 0
+        lo, n = src.range_start[along], src.range_end[along] - src.range_start[along] + 1
+        for q in range(patches):
+            dst = bc.face[bc.n_face]
+            bc.n_face += 1
+            for k, _ in L.Face._fields_:
+                setattr(dst, k, getattr(src, k))
+            dst.range_start[along], dst.range_end[along] = lo + n * q // patches, lo + n * (q + 1) // patches - 1
+    case.blocks[0].bc = bc
+    pr = Pair(case, precision=L.FP64)
+    pr.init()
+    for step in range(3):
+        e = max(pr.err("BV", halo=2), pr.err("SV", halo=2))
+        print(f"[gpu-small] after {step} steps: err {e:.2e}", flush=True)
+        assert e < 1e-9
+        pr.gpu.step()
+        pr.orc.step()
+    pr.close()
