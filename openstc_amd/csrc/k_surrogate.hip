@@ -197,8 +197,8 @@ struct TrainOut {
 struct InferOut {
   double *dy;                    // [n][9]
   unsigned *rejected;            // [n]: each workgroup's rejected cells (less its first cell), from its first cell on
-  unsigned *listed;              // [kSurRows]: cells in each workgroup's list
-  unsigned long long *stats;     // [stat_rows][4], a row per workgroup: its first cell, cells rejected for each reason
+  unsigned *listed;              // [kSurRows]: cells in each workgroup's list (list_of)
+  unsigned long long *stats;     // [stat_rows][4], a row per workgroup: cells rejected in all and for each reason
   int stat_rows;
   float *raw;                    // optional [n][16] standardised outputs
 };
@@ -231,6 +231,28 @@ __device__ __forceinline__ void save_layer(const TrainOut &tr, int l, long n, lo
 __device__ __forceinline__ int tile_l0(int mt) { return mt; }
 __device__ __forceinline__ int tile_h(int l, int mt, int kc) { return 8 + (l - 1) * 32 + mt * 4 + kc; }
 __device__ __forceinline__ int tile_out(int kc) { return 104 + kc; }
+
+// The forward's waves have equal runs of parts (16 * TILES cells), the first
+// `more` parts that are left over spread among them.
+struct Runs {
+  long each;
+  int more, waves, part;
+  __host__ __device__ Runs(long n, int part, int waves) : waves(waves), part(part) {
+    const long parts = (n + part - 1) / part;
+    each = parts / waves;
+    more = (int)(parts - each * waves);
+  }
+  __host__ __device__ long first_cell(int wave) const {
+    return (each * wave + (int)((unsigned)wave * (unsigned)more / (unsigned)waves)) * part;
+  }
+};
+
+// The lists' order: those of one XCD's workgroups (dealt round-robin to the 8
+// XCDs) one after the other, and back.
+__device__ __forceinline__ int list_of(int wg) { return (wg & 7) * (kSurRows / 8) + (wg >> 3); }
+__device__ __forceinline__ int workgroup_of(int list) {
+  return (list & (kSurRows / 8 - 1)) * 8 + list / (kSurRows / 8);
+}
 
 // The whole network for CELLS cells per wave pass (features one lane per cell,
 // then the layers for 16 * TILES cells at a time), and for inference the
@@ -266,19 +288,13 @@ __global__ __launch_bounds__(WAVES * 64) void k_sur_forward(SurParams s, Src src
 
   const int wave = threadIdx.x >> 6, ln = threadIdx.x & 63, g = ln >> 4, cn = ln & 15;
   const long n = src.n;
-  // each wave takes an equal run of parts (16 * TILES cells), up to CELLS
-  // cells a pass: with whole passes dealt out in turn the last round would
-  // leave most waves idle
+  // each wave takes its run, up to CELLS cells a pass: with whole passes dealt
+  // out in turn the last round would leave most waves idle
   constexpr int kPart = 16 * TILES;
-  const long parts = (n + kPart - 1) / kPart;
-  const int waves = (int)gridDim.x * WAVES, w = (int)blockIdx.x * WAVES + wave;
-  const long each = parts / waves;
-  const int more = (int)(parts - each * waves);  // waves with one part more, spread over the workgroups
-  auto first_cell = [&](int v) {
-    return (each * v + (int)((unsigned)v * (unsigned)more / (unsigned)waves)) * kPart;
-  };
-  const long wg0 = first_cell((int)blockIdx.x * WAVES), end = min(n, first_cell(w + 1));
-  for (long base = first_cell(w); base < end; base += CELLS) {
+  const int w = (int)blockIdx.x * WAVES + wave;
+  const Runs runs(n, kPart, (int)gridDim.x * WAVES);
+  const long wg0 = runs.first_cell((int)blockIdx.x * WAVES), end = min(n, runs.first_cell(w + 1));
+  for (long base = runs.first_cell(w); base < end; base += CELLS) {
     const int live = (int)min((long)CELLS, end - base);  // cells of this pass
     float *stg = sStage[wave];
     // ---- features, one lane per cell, as BF16 pairs in the cell's staging row
@@ -476,12 +492,11 @@ __global__ __launch_bounds__(WAVES * 64) void k_sur_forward(SurParams s, Src src
     // the workgroup's row, and the rows without a workgroup cleared
     __syncthreads();
     if (threadIdx.x < 4)
-      io.stats[(long)blockIdx.x * 4 + threadIdx.x] =
-          threadIdx.x == 0 ? (unsigned long long)wg0 : (unsigned long long)rejected[threadIdx.x];
-    if (threadIdx.x == 0) io.listed[blockIdx.x] = rejected[0];
+      io.stats[(long)blockIdx.x * 4 + threadIdx.x] = (unsigned long long)rejected[threadIdx.x];
+    if (threadIdx.x == 0) io.listed[list_of(blockIdx.x)] = rejected[0];
     if (blockIdx.x == 0) {
       for (int q = gridDim.x * 4 + threadIdx.x; q < io.stat_rows * 4; q += blockDim.x) io.stats[q] = 0;
-      for (int q = gridDim.x + threadIdx.x; q < kSurRows; q += blockDim.x) io.listed[q] = 0;
+      for (int q = gridDim.x + threadIdx.x; q < kSurRows; q += blockDim.x) io.listed[list_of(q)] = 0;
     }
   }
 }
@@ -504,18 +519,21 @@ __device__ __forceinline__ int touch_tables(const ostc_param *__restrict__ p, in
 // the waves take pieces of all workgroups' lists joined end to end, so that
 // neither a wave nor a round is partly filled.  Rejected cells come in clusters
 // (a list is a run of cells, in a zone a region of space): with waves bound to
-// a list, 2 % of a 256x192x128 zone in one region made a step of 2 617 us (1 251
+// a list, 2 % of a 256x192x128 zone in one region made a step of 2 587 us (1 247
 // with them spread out), since the waves of a few lists went round 48 times
-// while the others had none; now it is 1 225 us (1 234).  Every wave sums the
-// lists' lengths itself (four a lane and a wave scan).
+// while the others had none; now it is 1 203 us (1 215).  Every wave sums the
+// lists' lengths itself (four a lane and a wave scan) and finds a cell's list
+// by bisection, while the chemistry's tables are on their way.  The lists are
+// joined XCD by XCD: where they are alike, a wave finds its lists and states
+// in the L2 that the forward kernel left them in (300 000 states, most of them
+// rejected, 80 -> 77 us).
 template <typename Src, bool RED>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 : 1))) void k_sur_fallback(
     const ostc_param *__restrict__ p, Src src, const unsigned *__restrict__ rejected,
-    const unsigned *__restrict__ listed, const unsigned long long *__restrict__ stats, int rows,
+    const unsigned *__restrict__ listed, Runs runs, int waves_per_wg,
     double *__restrict__ dyo) {
   __shared__ ConcGibbs tab_mem[RED ? kRedEntries * 64 : 1];
   __shared__ __attribute__((aligned(16))) unsigned upto[kSurRows];  // cells in the lists up to this one
-  __shared__ long first[kSurRows];     // first cell of each list's workgroup
   static_assert(kSurRows == 4 * 64, "four lists a lane");
   const int ln = threadIdx.x;
   uint4 sum = reinterpret_cast<const uint4 *>(listed)[ln];
@@ -529,24 +547,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, RED ? 2 :
     if (ln >= d) at += below;
   }
   const unsigned total = (unsigned)__builtin_amdgcn_readlane((int)at, 63);
-  if (blockIdx.x * 64u >= total) return;
+  // the grid is a multiple of 8: the workgroups on one XCD share an eighth of
+  // the pieces, those of that XCD's own lists where the lists are alike
+  const unsigned pieces = (total + 63) / 64, x = blockIdx.x & 7;
+  const unsigned from = pieces * x / 8 + blockIdx.x / 8, to = pieces * (x + 1) / 8;
+  if (from >= to) return;
   at -= sum.w;
   reinterpret_cast<uint4 *>(upto)[ln] = make_uint4(at + sum.x, at + sum.y, at + sum.z, at + sum.w);
-#pragma unroll
-  for (int r = ln; r < kSurRows; r += 64) first[r] = r < rows ? (long)stats[(long)r * 4] : 0;
-  if constexpr (RED) {
-    const int warm = touch_tables(p, ln);
-    asm volatile("" ::"v"(warm));
-  }
+  int warm = 0;  // on its way while the wave looks for its cells
+  if constexpr (RED) warm = touch_tables(p, ln);
   wave_sync();
-  for (unsigned q = blockIdx.x * 64u + ln; q < total; q += gridDim.x * 64u) {
+  for (unsigned piece = from; piece < to; piece += gridDim.x / 8) {
+    const unsigned q = piece * 64 + ln;
+    if (q >= total) break;
     int l = 0;  // the list of entry q: lists whose cells all come before it
 #pragma unroll
     for (int d = kSurRows / 2; d > 0; d /= 2)
       if (upto[l + d - 1] <= q) l += d;
-    const long wg0 = first[l], c = wg0 + rejected[wg0 + (q - (l ? upto[l - 1] : 0u))];
+    const long wg0 = runs.first_cell(workgroup_of(l) * waves_per_wg);
+    const long c = wg0 + rejected[wg0 + (q - (l ? upto[l - 1] : 0u))];
     double T, P, DT, Y[kNs];
     src.load(c, T, P, Y, DT);
+    if constexpr (RED) asm volatile("" ::"v"(warm));
     if constexpr (RED) {
       plain_chem_step_red(p, T, P, Y, DT, tab_mem + ln, 64, [&](int k, double v) { dyo[c * kNs + k] = v; });
     } else {
@@ -759,7 +781,7 @@ int sur_pack(const SurState &st, hipStream_t s) {
 }
 
 template <typename Src, bool TRAIN, int CELLS, int TILES, int WAVES>
-static void launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
+static Runs launch_forward(const SurState &st, const Src &src, const TrainOut &tr, const InferOut &io,
                            hipStream_t s) {
   const long wgs = (src.n + WAVES * CELLS - 1) / (WAVES * CELLS);
   const dim3 grid((unsigned)std::max<long>(1, std::min<long>(wgs, st.cus))), block(WAVES * 64);
@@ -770,6 +792,7 @@ static void launch_forward(const SurState &st, const Src &src, const TrainOut &t
   else
     hipLaunchKernelGGL((k_sur_forward<Src, TRAIN, OSTC_SUR_GELU, CELLS, TILES, WAVES>), grid, block, 0, s,
                        st.params, src, wpk, st.bias, tr, io);
+  return Runs(src.n, 16 * TILES, (int)grid.x * WAVES);
 }
 
 template <typename Src>
@@ -778,19 +801,19 @@ static int infer_impl(const SurState &st, const ostc_param *dp, bool red, const 
   TrainOut tr{};
   InferOut io{dy, st.rejected, st.listed, st.stats, st.cus, raw};
   // batches that 64-cell passes would leave on part of the CUs: 16 cells a wave
-  if (src.n < 64L * kWaves * st.cus / 2)
-    launch_forward<Src, false, 16, 1, 4>(st, src, tr, io, s);
-  else
-    launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
+  const bool few = src.n < 64L * kWaves * st.cus / 2;
+  const Runs runs = few ? launch_forward<Src, false, 16, 1, 4>(st, src, tr, io, s)
+                        : launch_forward<Src, false, 64, 2, kWaves>(st, src, tr, io, s);
   // one wave per 64 cells, as many as the registers let the device hold (two
-  // or one a SIMD); those past the number rejected end at once
-  const dim3 fb_grid((unsigned)std::min<long>((src.n + 63) / 64, (red ? 8L : 4L) * st.cus));
+  // or one a SIMD), a multiple of the XCDs; those past the number rejected end
+  // at once
+  const dim3 fb_grid((unsigned)std::min<long>((src.n + 511) / 512, (red ? 8L : 4L) * st.cus / 8) * 8);
   if (red)
     hipLaunchKernelGGL((k_sur_fallback<Src, true>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.listed,
-                       st.stats, st.cus, dy);
+                       runs, few ? 4 : kWaves, dy);
   else
     hipLaunchKernelGGL((k_sur_fallback<Src, false>), fb_grid, dim3(64), 0, s, dp, src, st.rejected, st.listed,
-                       st.stats, st.cus, dy);
+                       runs, few ? 4 : kWaves, dy);
   return hipGetLastError() == hipSuccess ? OSTC_OK : OSTC_ERR_HIP;
 }
 

@@ -61,7 +61,7 @@ struct SurState {
   unsigned *rejected = nullptr;  // [fb_cap] cells the checks rejected, by forward workgroup
   long fb_cap = 0;               // cells `rejected` is sized for
   unsigned *listed = nullptr;    // [kSurRows] cells in each list
-  unsigned long long *stats = nullptr;  // [cus][4], a row per workgroup: its first cell, cells rejected by reason
+  unsigned long long *stats = nullptr;  // [cus][4], a row per workgroup: cells rejected in all and by reason
   // training buffers (max_batch rows)
   float *a0 = nullptr, *z = nullptr, *a = nullptr, *yout = nullptr, *g5 = nullptr;
   float *gbuf[2] = {nullptr, nullptr};
